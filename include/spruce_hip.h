@@ -318,6 +318,18 @@ int spruce_gate_project_levels(const void* const* levels, const int64_t* level_n
                                void* stream);
 
 /*
+ * spruce_gate_project_levels for L layers in one launch, each with its own
+ * weights: level v's buffer holds [L, S, level_nodes[v], Pk, D], w is
+ * [L, D, P] (FlatGate's parameter) and out [L, S, N, Pk, P] or its
+ * interleaved form per layer.  The values of L calls, one per layer.
+ * Replaces FlatGate.project_queries / project_keys over a whole model's
+ * features (selector/gate.py:120-127).  1 <= L < 65536.
+ */
+int spruce_gate_project_layers(const void* const* levels, const int64_t* level_nodes, int64_t nlevels, int64_t L,
+                               int64_t S, int64_t Pk, int64_t D, int dtype, const float* w, int64_t P, float* out,
+                               int layout, void* stream);
+
+/*
  * MaxSim block scores: scores[s][i][j] = max over prototype pairs (a, c) of
  * qp[s][i][a] . kp[s][j][c], divided by div (= sqrt(P)).  causal = 1: only
  * j <= i is computed and j > i is written as -inf; causal = 2 with Qb == Kb:

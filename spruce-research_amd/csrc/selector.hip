@@ -27,6 +27,8 @@
 // The pooling kernel streams Q and K once from HBM (the dominant cost of the
 // front end: Q is 7x the bytes of K at 28/4 heads); the rest touches only the
 // pooled summaries and the [Qb, Kb] score matrix.
+#include <type_traits>
+
 #include "common.h"
 
 namespace spruce {
@@ -502,20 +504,38 @@ __global__ __launch_bounds__(256) void project_tile_kernel(const ProjPair pp) {
   }
 }
 
-// Large-N form of the kernel above: a TR x TC register tile per thread
-// (16 x 16 threads, a 16TR x 16TC output tile per workgroup) and d staged in
-// slices of kBD, so each step reads TR / 4 + TC / 4 float4 from LDS for
-// TR * TC FMAs (8 x 4: 96 bytes per FMA instruction against 128 for 4 x 4,
-// whose reads alone keep the LDS busy). Same fmaf chain per output (d in
-// order from 0), so the results are identical. Requires D % 4 == 0,
-// P % 4 == 0 and 16-byte aligned operands.
-constexpr int kBD = 32;
-// 8 x 4 per thread from 16K rows (fewer rows leave CUs idle with 128-row
-// tiles). Measured at p = d = 128: N = 131072 0.102 -> 0.068 ms, N = 65536
-// 0.056 -> 0.039 ms; 8 x 8 and 4 x 8 within 5% of 8 x 4.
-constexpr int kBlockProjectRows = 16384, kBlockProjectTR = 8, kBlockProjectTC = 4;
+// ---------------------------------------------------------------------------
+// Float32 contractions on the matrix cores.  v_mfma_f32_32x32x2_f32 adds its
+// two products to an accumulator one after the other, each with a single
+// rounding, so a sequence of them over e = 0, 2, 4, ... is the fmaf chain of
+// the projections and scores, bit for bit (compared on the GPU over normal,
+// wide-exponent, denormal and special operands); it reaches 155 TFLOP/s where
+// unpacked VALU fmaf chains reach 79.  (The 32x32x1 form takes operands as
+// stored but reaches 135: twice the accumulator traffic.)
+// Lane l supplies row l % 32 of A and column l % 32 of B at e + l / 32, so a
+// staged row keeps the even e of each 8 before the odd ones and a lane reads
+// the operands of four steps as 16 bytes.  Accumulator element r: row
+// 8 (r / 4) + 4 (lane / 32) + r % 4, column lane % 32.
+constexpr int kMS = 32, kMRow = kMS + 4;  // slice of the contracted dim; padded LDS row (conflict-free reads)
 
-// Input rows of project_block_kernel: row n of one contiguous float32 [N, D]
+// Stores e = 4 c4 .. 4 c4 + 3 of staged row r.
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void stage_even_odd(float* rows, int r, int c4, f32x4_t v) {
+  float* o = rows + r * kMRow + 8 * (c4 >> 1) + 2 * (c4 & 1);
+  *reinterpret_cast<f32x2_t*>(o) = f32x2_t{v[0], v[2]};
+  *reinterpret_cast<f32x2_t*>(o + 4) = f32x2_t{v[1], v[3]};
+}
+
+__device__ __forceinline__ f32x16_t mfma_f32(float a, float b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+
+// Workgroup id -> position: consecutive ids go round-robin to the 8 XCDs, so
+// each XCD takes one contiguous eighth of the positions and its L2 keeps the
+// operands that neighbouring tiles share.  The grid is padded to 8 * per.
+__device__ __forceinline__ int64_t xcd_chunk(int64_t bid, int64_t per) { return (bid & 7) * per + (bid >> 3); }
+
+// Input rows of project_mfma_kernel: row n of one contiguous float32 [N, D]
 // buffer ...
 struct ProjRowsF32 {
   const float* x;
@@ -547,143 +567,177 @@ struct ProjRowsSeg {
   }
 };
 
-// Four consecutive input values at element e of a row, widened to float32.
-__device__ __forceinline__ float4 load4_row(const ProjRowsF32&, const void* row, int e) {
-  return *reinterpret_cast<const float4*>(static_cast<const float*>(row) + e);
+// Four consecutive input values at element e of a row as loaded, and widened to float32.
+__device__ __forceinline__ f32x4_t load4_raw(const ProjRowsF32&, const void* row, int e) {
+  return *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(row) + e);
 }
+__device__ __forceinline__ f32x4_t widen4(const ProjRowsF32&, f32x4_t v) { return v; }
 template <typename TIn>
-__device__ __forceinline__ float4 load4_row(const ProjRowsSeg<TIn>&, const void* row, int e) {
+__device__ __forceinline__ auto load4_raw(const ProjRowsSeg<TIn>&, const void* row, int e) {
+  if constexpr (TIn::bytes == 4)
+    return *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(row) + e);
+  else
+    return *reinterpret_cast<const u32x2_t*>(static_cast<const uint16_t*>(row) + e);
+}
+template <typename TIn, typename V>
+__device__ __forceinline__ f32x4_t widen4(const ProjRowsSeg<TIn>&, V w) {
   if constexpr (TIn::bytes == 4) {
-    return *reinterpret_cast<const float4*>(static_cast<const float*>(row) + e);
+    return w;
   } else {
     constexpr bool F16 = TIn::code == SPRUCE_DTYPE_F16;
-    const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(row) + e);
-    return float4{unpack1<F16>(w.x & 0xffffu), unpack1<F16>(w.x >> 16), unpack1<F16>(w.y & 0xffffu),
-                  unpack1<F16>(w.y >> 16)};
+    return f32x4_t{unpack1<F16>(w[0] & 0xffffu), unpack1<F16>(w[0] >> 16), unpack1<F16>(w[1] & 0xffffu),
+                   unpack1<F16>(w[1] >> 16)};
   }
 }
 
+// Projections as one matrix product: a workgroup of 2 x 2 waves covers
+// 64 RA x 128 outputs, each wave 32 RA x 64, in slices of 32 d (the next
+// slice's loads are in flight during the current one's products).  blockIdx.z is the layer: `rows` rows of x, its own [D, P]
+// weights.
 // IL: rows are (node, prototype) pairs with ilk prototypes per node, and out
 // is [nodes, P/4, ilk, 4] (each node's prototypes interleaved by 4-column
-// group) instead of [N, P]; the output tile goes through LDS so that
+// group) instead of [N, P].  The operands then change sides (A = columns of
+// w), so that a lane holds four neighbouring columns of one row and
 // neighbouring lanes store neighbouring 16-byte slots.
-template <int TR, int TC, typename Rows, bool IL = false>
-__global__ __launch_bounds__(256) void project_block_kernel(const Rows src, const float* __restrict__ w, int64_t N,
-                                                            int D, int P, float* __restrict__ out, int ilk = 0) {
-  constexpr int R = 16 * TR, C = 16 * TC;          // workgroup tile
-  constexpr int XL = R * kBD / 4 / 256;            // x float4 per thread per slice
-  constexpr int WL = C * kBD / 4 / 256;            // w float4 per thread per slice
-  constexpr int kXs = kBD * (R + 4), kWs = kBD * C, kOut = IL ? R * (C + 4) : 0;
-  __shared__ __attribute__((aligned(16))) float smem[kXs + kWs > kOut ? kXs + kWs : kOut];
-  float (*xs)[R + 4] = reinterpret_cast<float (*)[R + 4]>(smem);
-  float (*ws)[C] = reinterpret_cast<float (*)[C]>(smem + kXs);
-  const int tid = threadIdx.x;
-  const int tr = tid >> 4, tc = tid & 15;
-  const int64_t n0 = (int64_t)blockIdx.x * R;
+// Requires D % 4 == 0, P % 4 == 0 and 16-byte aligned operands.
+//
+// Bound: fp32 MFMA issue, after each tile's loads and before its float32
+// stores.  D = P = 128, bf16 rows: 28 layers of 4096 rows, both sides, 56
+// launches of 20 us (8 x 4 outputs a thread) and two stacking copies, 1164 us
+// -> two launches, 121 us; 131,040 node rows interleaved 85 -> 62 us.
+// From 16384 rows the 128-column tiles fill the CUs; fewer float32 rows of one
+// layer take the 64-column tiles above.
+constexpr int kMfmaProjectRows = 16384;
+template <int RA, typename Rows, bool IL>
+__global__ __launch_bounds__(256, RA == 2 ? 3 : 4) void project_mfma_kernel(const Rows src, const float* __restrict__ w,
+                                                                            int64_t rows, int D, int P,
+                                                                            float* __restrict__ out, int ilk) {
+  constexpr int R = IL ? 128 : 64 * RA, C = IL ? 64 * RA : 128;  // rows of x, columns of w per workgroup
+  constexpr int XL = R * kMS / 4 / 256, WL = C * kMS / 4 / 256;  // groups of 4 d per thread per slice
+  __shared__ __attribute__((aligned(16))) float xs[R * kMRow];
+  __shared__ __attribute__((aligned(16))) float ws[C * kMRow];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wr = __builtin_amdgcn_readfirstlane(tid >> 7), wc = __builtin_amdgcn_readfirstlane((tid >> 6) & 1);
+  const int64_t n0 = (int64_t)blockIdx.x * R, base = (int64_t)blockIdx.z * rows;
   const int j0 = blockIdx.y * C;
-  float acc[TR][TC];
-#pragma unroll
-  for (int a = 0; a < TR; ++a)
-#pragma unroll
-    for (int c = 0; c < TC; ++c) acc[a][c] = 0.f;
-  // The rows this thread stages are the same in every slice.
+  const int c4 = tid & 7;
+  // The rows this thread stages are the same in every slice.  Rows, dims and
+  // columns past the end read the last one instead (unconditional loads stay
+  // in flight together; nothing computed from them is stored).  w is read
+  // along its rows: thread tid takes column tid % C, 4 d at a time.
   const void* xrow[XL];
 #pragma unroll
-  for (int t = 0; t < XL; ++t) {
-    const int64_t n = n0 + (tid + 256 * t) / (kBD / 4);
-    xrow[t] = n < N ? src.row(n, D) : nullptr;
+  for (int u = 0; u < XL; ++u) {
+    const int64_t n = n0 + (tid >> 3) + 32 * u;
+    xrow[u] = src.row(base + (n < rows ? n : rows - 1), D);
   }
-  for (int d0 = 0; d0 < D; d0 += kBD) {
-    const int dn = D - d0 < kBD ? D - d0 : kBD;
-    float4 xv[XL], wv[WL];
+  const int wcol = tid % C, wd4 = tid / C;
+  const float* wp = w + (int64_t)blockIdx.z * D * P + (j0 + wcol < P ? j0 + wcol : P - 1);
+  decltype(load4_raw(src, nullptr, 0)) xv[XL];
+  f32x4_t wv[WL];
+  auto load_slice = [&](int d0) {
+    const int xd = d0 + 4 * c4 < D ? d0 + 4 * c4 : D - 4;
 #pragma unroll
-    for (int t = 0; t < XL; ++t) {
-      const int c4 = (tid + 256 * t) % (kBD / 4);
-      xv[t] = (xrow[t] != nullptr && 4 * c4 < dn) ? load4_row(src, xrow[t], d0 + 4 * c4)
-                                                   : float4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int u = 0; u < XL; ++u) xv[u] = load4_raw(src, xrow[u], xd);
 #pragma unroll
-    for (int t = 0; t < WL; ++t) {
-      const int e = tid + 256 * t, dd = e / (C / 4), c4 = e % (C / 4);
-      const int j = j0 + 4 * c4;
-      wv[t] = (dd < dn && j < P) ? *reinterpret_cast<const float4*>(w + (int64_t)(d0 + dd) * P + j)
-                                 : float4{0.f, 0.f, 0.f, 0.f};
-    }
-    if (d0 > 0) __syncthreads();  // the previous slice's reads are done
+    for (int u = 0; u < WL; ++u) {
+      int d = d0 + 4 * (wd4 + 256 / C * u);
+      d = d < D ? d : D - 4;
 #pragma unroll
-    for (int t = 0; t < XL; ++t) {
-      const int e = tid + 256 * t, r = e / (kBD / 4), c4 = e % (kBD / 4);
-      xs[4 * c4][r] = xv[t].x;
-      xs[4 * c4 + 1][r] = xv[t].y;
-      xs[4 * c4 + 2][r] = xv[t].z;
-      xs[4 * c4 + 3][r] = xv[t].w;
+      for (int e = 0; e < 4; ++e) wv[u][e] = wp[(int64_t)(d + e) * P];
     }
+  };
+  auto store_slice = [&]() {
 #pragma unroll
-    for (int t = 0; t < WL; ++t) {
-      const int e = tid + 256 * t, dd = e / (C / 4), c4 = e % (C / 4);
-      *reinterpret_cast<float4*>(&ws[dd][4 * c4]) = wv[t];
-    }
+    for (int u = 0; u < XL; ++u) stage_even_odd(xs, (tid >> 3) + 32 * u, c4, widen4(src, xv[u]));
+#pragma unroll
+    for (int u = 0; u < WL; ++u) stage_even_odd(ws, wcol, wd4 + 256 / C * u, wv[u]);
+  };
+  f32x16_t acc[RA][2];
+#pragma unroll
+  for (int a = 0; a < RA; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+  const float* as = (IL ? ws : xs) + (wr * 32 * RA + (lane & 31)) * kMRow + 4 * (lane >> 5);
+  const float* bs = (IL ? xs : ws) + (wc * 64 + (lane & 31)) * kMRow + 4 * (lane >> 5);
+  // Pairs of d from d = 8 g of the slice (4 of them, or 2 in a tail).
+  auto group = [&](int g, auto steps) {
+    f32x4_t av[RA], bv[2];
+#pragma unroll
+    for (int a = 0; a < RA; ++a) av[a] = *reinterpret_cast<const f32x4_t*>(as + 32 * a * kMRow + 8 * g);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) bv[b] = *reinterpret_cast<const f32x4_t*>(bs + 32 * b * kMRow + 8 * g);
+#pragma unroll
+    for (int s = 0; s < decltype(steps)::value; ++s)
+#pragma unroll
+      for (int a = 0; a < RA; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = mfma_f32(av[a][s], bv[b][s], acc[a][b]);
+  };
+  load_slice(0);
+  int d0 = 0;
+  for (; d0 + kMS <= D; d0 += kMS) {
+    __syncthreads();  // the previous slice has been read
+    store_slice();
     __syncthreads();
-#pragma unroll 2
-    for (int dd = 0; dd < dn; ++dd) {
-      float av[TR], bv[TC];
+    if (d0 + kMS < D) load_slice(d0 + kMS);
 #pragma unroll
-      for (int a = 0; a < TR; a += 4) {
-        const float4 a4 = *reinterpret_cast<const float4*>(&xs[dd][TR * tr + a]);
-        av[a] = a4.x;
-        av[a + 1] = a4.y;
-        av[a + 2] = a4.z;
-        av[a + 3] = a4.w;
-      }
-#pragma unroll
-      for (int c = 0; c < TC; c += 4) {
-        const float4 b4 = *reinterpret_cast<const float4*>(&ws[dd][TC * tc + c]);
-        bv[c] = b4.x;
-        bv[c + 1] = b4.y;
-        bv[c + 2] = b4.z;
-        bv[c + 3] = b4.w;
-      }
-#pragma unroll
-      for (int a = 0; a < TR; ++a)
-#pragma unroll
-        for (int c = 0; c < TC; ++c) acc[a][c] = __builtin_fmaf(av[a], bv[c], acc[a][c]);
-    }
+    for (int g = 0; g < kMS / 8; ++g) group(g, std::integral_constant<int, 4>{});
   }
-  if constexpr (IL) {
-    // Tile [R][C + 4] in LDS, then slot s = (group g, row) with the row
-    // fastest: consecutive rows of a node are consecutive 16-byte slots of
-    // out (value (n, j) at node * ilk * P + (j / 4) * 4 * ilk + proto * 4).
-    constexpr int OS = C + 4;
-    __syncthreads();  // every read of xs / ws is done
-#pragma unroll
-    for (int a = 0; a < TR; ++a)
-#pragma unroll
-      for (int c = 0; c < TC; c += 4)
-        *reinterpret_cast<float4*>(&smem[(TR * tr + a) * OS + TC * tc + c]) =
-            float4{acc[a][c], acc[a][c + 1], acc[a][c + 2], acc[a][c + 3]};
+  if (d0 < D) {
     __syncthreads();
-    for (int sl = tid; sl < R * (C / 4); sl += 256) {
-      const int row = sl % R, g = sl / R;
-      const int64_t n = n0 + row;
-      const int j = j0 + 4 * g;
-      if (n >= N || j >= P) continue;
-      const int64_t node = n / ilk;
-      *reinterpret_cast<float4*>(out + node * ilk * P + (int64_t)(j / 4) * 4 * ilk + (n - node * ilk) * 4) =
-          *reinterpret_cast<const float4*>(&smem[row * OS + 4 * g]);
-    }
-  } else {
+    store_slice();
+    __syncthreads();
+    for (int g = 0; g < (D - d0) / 8; ++g) group(g, std::integral_constant<int, 4>{});
+    if ((D - d0) % 8) group((D - d0) / 8, std::integral_constant<int, 2>{});
+  }
 #pragma unroll
-    for (int a = 0; a < TR; ++a) {
-      const int64_t n = n0 + TR * tr + a;
-      if (n >= N) continue;
+  for (int b = 0; b < 2; ++b) {
+    if constexpr (IL) {
+      const int64_t n = n0 + wc * 64 + 32 * b + (lane & 31);
+      if (n >= rows) continue;
+      const int64_t node = (base + n) / ilk;
+      float* o = out + node * ilk * P + (base + n - node * ilk) * 4;
 #pragma unroll
-      for (int c = 0; c < TC; c += 4) {
-        const int j = j0 + TC * tc + c;
-        if (j < P)
-          *reinterpret_cast<float4*>(out + n * P + j) = float4{acc[a][c], acc[a][c + 1], acc[a][c + 2], acc[a][c + 3]};
-      }
+      for (int a = 0; a < RA; ++a)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+          const int j = j0 + wr * 32 * RA + 32 * a + 2 * r + 4 * (lane >> 5);
+          if (j < P)
+            *reinterpret_cast<float4*>(o + (int64_t)j * ilk) = float4{acc[a][b][r], acc[a][b][r + 1], acc[a][b][r + 2],
+                                                                      acc[a][b][r + 3]};
+        }
+    } else {
+      const int j = j0 + wc * 64 + 32 * b + (lane & 31);
+      if (j >= P) continue;
+#pragma unroll
+      for (int a = 0; a < RA; ++a)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int64_t n = n0 + wr * 32 * RA + 32 * a + 8 * (r / 4) + 4 * (lane >> 5) + r % 4;
+          if (n < rows) out[(base + n) * P + j] = acc[a][b][r];
+        }
     }
   }
+}
+
+// Launches project_mfma_kernel over L layers of `rows` rows each.
+template <typename Rows>
+int launch_project_mfma(const Rows& src, const float* w, int64_t L, int64_t rows, int D, int P, float* out, bool il,
+                        int ilk, hipStream_t st) {
+  // 128 x 128 tiles once they give every CU about two workgroups.
+  const int64_t big = L * ((rows + 127) / 128) * ((P + 127) / 128);
+  auto go = [&](auto kernel, int R, int C) {
+    const int64_t gx = (rows + R - 1) / R, gy = (P + C - 1) / C;
+    SPRUCE_REQUIRE(gx < ((int64_t)1 << 31) && gy < 65536 && L < 65536, "projection too large");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)gy, (unsigned)L), dim3(256), 0, st, src, w, rows, D, P, out,
+                       ilk);
+    return check_launch("project_mfma_kernel");
+  };
+  if (il) return big >= 512 ? go(project_mfma_kernel<2, Rows, true>, 128, 128) : go(project_mfma_kernel<1, Rows, true>, 128, 64);
+  return big >= 512 ? go(project_mfma_kernel<2, Rows, false>, 128, 128) : go(project_mfma_kernel<1, Rows, false>, 64, 128);
 }
 
 // MaxSim scores over a tile of 16 query blocks x 64 key blocks: lane = key
@@ -785,157 +839,187 @@ __global__ __launch_bounds__(256) void gate_scores_kernel(const ScoreParams p) {
   }
 }
 
-// The same scores, register-blocked, for one query prototype and PK (1 or 2)
-// key prototypes: a workgroup covers 16TR query blocks x 64 key blocks and
-// thread (tr, tc) holds query blocks TR*tr..TR*tr+TR-1 x key blocks
-// 4tc..4tc+3 for every key prototype. The prototypes are staged transposed
-// ([e][block]) in slices of kGS dims, so each step over e reads TR query
-// values and PK float4 of key values for 4 * TR * PK fmaf (the kernel above
-// reads five float4 for 16). Same operation order as the kernel above.
-constexpr int kGT = 64, kGS = 32;  // key tile, slice of the projection dim
-constexpr int kScoreTR = 2;        // query blocks per thread (tile of 16 * kScoreTR)
-template <int PK, int TR>
-__global__ __launch_bounds__(256) void gate_scores_tile_kernel(const ScoreParams p) {
-  constexpr int R = 16 * TR;               // query blocks per tile
-  constexpr int kXRow = R + 4, kYRow = kGT + 4;  // padded LDS rows (floats)
-  constexpr int kBands = kGT / R;          // query tiles per 64-block band
-  __shared__ __attribute__((aligned(16))) float xs[kGS * kXRow];
-  __shared__ __attribute__((aligned(16))) float ys[PK * kGS * kYRow];
-  int bg, i0, j0;
-  if (p.causal == 2) {
-    // 1-D grid over the tiles on or below the diagonal (Qb == Kb).  Band m
-    // (query blocks 64m..64m+63) holds kBands query tiles of m + 1 key tiles
-    // each, kBands * m(m+1)/2 tiles before it.
-    const int nt = (p.Qb + kGT - 1) / kGT, ntri = kBands * (nt * (nt + 1) / 2);
-    bg = blockIdx.x / ntri;
-    const int t = blockIdx.x - bg * ntri;
-    int m = (int)((sqrtf(8.f * (float)t / kBands + 1.f) - 1.f) * 0.5f);
-    while (kBands * ((m + 1) * (m + 2) / 2) <= t) ++m;
-    while (kBands * (m * (m + 1) / 2) > t) --m;
-    const int rem = t - kBands * (m * (m + 1) / 2);
-    const int h = rem / (m + 1);
-    i0 = (m * kBands + h) * R;
-    j0 = (rem - h * (m + 1)) * kGT;
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float x) {
+  return fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true)));
+}
+
+// The scores above for 1, 2, 4 or 8 prototypes a side, as one matrix product
+// of prototype rows: a workgroup of 2 x 2 waves covers 64 RA query rows x 128
+// key rows, each wave 32 RA x 64, and reduces its accumulators to one maximum
+// per (query block, key block): the PQ rows of a query block are registers of
+// one lane (and its other half for PQ = 8), the PK columns neighbouring lanes.
+// fmaxf drops NaN as "replace when strictly larger" does, except for the
+// first pair, which the writing lane holds itself and keeps if it is NaN; a
+// maximum of exactly zero may take either sign.
+//
+// Bound: fp32 MFMA issue (busy 68% of the cycles; three waves a SIMD, the
+// rest is each tile's first loads and its reduction).  8 x 8 prototypes,
+// 28 x 2 slabs of 256 x 256 blocks, causal: 10.17 ms with one thread per
+// score (every pair a dependent chain whose operands come through the cache)
+// -> 0.319 ms.  One query and two key prototypes, 4 slabs of 1024 blocks:
+// 31.9 (VALU, 2 x 4 x 2 outputs a thread) -> 23.8 us.
+template <int PQ, int PK, int RA>
+__global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate_scores_mfma_kernel(const ScoreParams p, int nti, int ntj,
+                                                                                int64_t slab_tiles, int64_t tiles,
+                                                                                int64_t per) {
+  constexpr int TM = 64 * RA, TN = 128, TI = TM / PQ, TJ = TN / PK;
+  constexpr int XL = TM * kMS / 4 / 256, YL = TN * kMS / 4 / 256;  // float4 per thread per slice
+  __shared__ __attribute__((aligned(16))) float xs[TM * kMRow];
+  __shared__ __attribute__((aligned(16))) float ys[TN * kMRow];
+  const int64_t id = xcd_chunk(blockIdx.x, per);
+  if (id >= tiles) return;
+  const int64_t bg = id / slab_tiles;
+  const int t = (int)(id - bg * slab_tiles);
+  int ti, tj;
+  const bool tri = slab_tiles != (int64_t)nti * ntj;
+  if (tri) {
+    // Qb == Kb: row tile m holds the column tiles that reach the diagonal,
+    // kQ (m + 1) of them (TI >= TJ) or m / kB + 1 (TI < TJ), and the tiles
+    // before it are counted by `before`.
+    constexpr int kQ = TI >= TJ ? TI / TJ : 1, kB = TI >= TJ ? 1 : TJ / TI;
+    auto before = [](int m) {
+      const int64_t a = m / kB, r = m - a * kB;
+      return kQ * (kB * (a * (a + 1) / 2) + r * (a + 1));
+    };
+    ti = (int)sqrtf(2.f * (float)t * kB / kQ);
+    ti = ti < nti ? ti : nti - 1;
+    while (before(ti + 1) <= t) ++ti;
+    while (before(ti) > t) --ti;
+    tj = t - (int)before(ti);
   } else {
-    bg = blockIdx.z;
-    i0 = blockIdx.x * R;
-    j0 = blockIdx.y * kGT;
+    ti = t / ntj;
+    tj = t - ti * ntj;
   }
-  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
-  float* out = p.scores + (int64_t)bg * p.Qb * p.Kb;
-  if (p.causal && j0 > i0 + R - 1) {
+  const int i0 = ti * TI, j0 = tj * TJ;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wr = __builtin_amdgcn_readfirstlane(tid >> 7), wc = __builtin_amdgcn_readfirstlane((tid >> 6) & 1);
+  float* out = p.scores + bg * p.Qb * p.Kb;
+  if (j0 >= p.Kb) return;  // the last row tile of a triangle may reach past the matrix
+  if (p.causal && j0 > i0 + TI - 1) {
     // Entirely above the diagonal.
-    for (int r = 0; r < TR; ++r) {
-      const int i = i0 + TR * tr + r;
-      for (int k = 0; k < 4; ++k) {
-        const int j = j0 + 4 * tc + k;
+    if (p.causal == 1)
+      for (int e = tid; e < TI * TJ; e += 256) {
+        const int i = i0 + e / TJ, j = j0 + e % TJ;
         if (i < p.Qb && j < p.Kb) out[(int64_t)i * p.Kb + j] = -INFINITY;
       }
-    }
     return;
   }
-  const float* qsrc = p.qp + (int64_t)bg * p.Qb * p.P;
-  const float* ksrc = p.kp + (int64_t)bg * p.Kb * PK * p.P;
-  float acc[PK][TR][4];
+  if (tri && p.causal == 1 && j0 + TJ > i0 + TI - 1) {
+    // The row tile's last column tile also fills what lies to its right.
+    const int rows = p.Qb - i0 < TI ? p.Qb - i0 : TI;
+    for (int r = tid >> 6; r < rows; r += 4)
+      for (int j = j0 + TJ + lane; j < p.Kb; j += 64) out[(int64_t)(i0 + r) * p.Kb + j] = -INFINITY;
+  }
+  // A wave whose outputs all lie above the diagonal or outside the matrix only stages.
+  const int iw = i0 + wr * 32 * RA / PQ, jw = j0 + wc * 64 / PK;
+  const bool live = iw < p.Qb && jw < p.Kb && !(p.causal && jw > iw + 32 * RA / PQ - 1);
+  const float* qsrc = p.qp + (bg * p.Qb + i0) * PQ * (int64_t)p.P;
+  const float* ksrc = p.kp + (bg * p.Kb + j0) * PK * (int64_t)p.P;
+  const int nq = (p.Qb - i0 < TI ? p.Qb - i0 : TI) * PQ;  // real rows of the tile
+  const int nk = (p.Kb - j0 < TJ ? p.Kb - j0 : TJ) * PK;
+  // Rows and dims past the end read the last one instead (unconditional
+  // loads stay in flight together; nothing computed from them is stored).
+  f32x4_t xv[XL], yv[YL];
+  const float *xp[XL], *yp[YL];
+  const int c4 = tid & 7;
 #pragma unroll
-  for (int c = 0; c < PK; ++c)
+  for (int u = 0; u < XL; ++u) {
+    const int r = (tid >> 3) + 32 * u;
+    xp[u] = qsrc + (int64_t)(r < nq ? r : nq - 1) * p.P;
+  }
 #pragma unroll
-    for (int r = 0; r < TR; ++r)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) acc[c][r][k] = 0.f;
-  // Staging map: kD4 consecutive lanes read one block's slice (contiguous).
-  constexpr int kD4 = kGS / 4;                  // float4 per block slice
-  constexpr int kLoadsQ = R * kD4 / 256;        // query float4 per thread
-  constexpr int kLoads = kGT * kD4 / 256;       // key float4 per thread per prototype
-  // The next slice's operands are loaded into registers while the current
-  // slice is consumed from LDS.
-  float4 qv[kLoadsQ], kv[PK][kLoads];
+  for (int u = 0; u < YL; ++u) {
+    const int r = (tid >> 3) + 32 * u;
+    yp[u] = ksrc + (int64_t)(r < nk ? r : nk - 1) * p.P;
+  }
   auto load_slice = [&](int e0) {
+    const int e = e0 + 4 * c4 < p.P ? e0 + 4 * c4 : p.P - 4;
 #pragma unroll
-    for (int t = 0; t < kLoadsQ; ++t) {
-      const int idx = tid + 256 * t, blk = idx / kD4, d4 = idx % kD4;
-      const int i = i0 + blk;
-      qv[t] = i < p.Qb ? *reinterpret_cast<const float4*>(qsrc + (int64_t)i * p.P + e0 + 4 * d4)
-                       : float4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int u = 0; u < XL; ++u) xv[u] = *reinterpret_cast<const f32x4_t*>(xp[u] + e);
 #pragma unroll
-    for (int t = 0; t < kLoads; ++t) {
-      const int idx = tid + 256 * t, blk = idx / kD4, d4 = idx % kD4;
-      const int j = j0 + blk;
+    for (int u = 0; u < YL; ++u) yv[u] = *reinterpret_cast<const f32x4_t*>(yp[u] + e);
+  };
+  auto store_slice = [&]() {
 #pragma unroll
-      for (int c = 0; c < PK; ++c)
-        kv[c][t] = j < p.Kb ? *reinterpret_cast<const float4*>(ksrc + ((int64_t)j * PK + c) * p.P + e0 + 4 * d4)
-                            : float4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int u = 0; u < XL; ++u) stage_even_odd(xs, (tid >> 3) + 32 * u, c4, xv[u]);
+#pragma unroll
+    for (int u = 0; u < YL; ++u) stage_even_odd(ys, (tid >> 3) + 32 * u, c4, yv[u]);
+  };
+  f32x16_t acc[RA][2];
+#pragma unroll
+  for (int a = 0; a < RA; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
+  const int xoff = (wr * 32 * RA + (lane & 31)) * kMRow + 4 * (lane >> 5);
+  const int yoff = (wc * 64 + (lane & 31)) * kMRow + 4 * (lane >> 5);
+  // Pairs of e from e = 8 g of the slice (4 of them, or 2 in a tail).
+  auto group = [&](int g, auto steps) {
+    f32x4_t x[RA], y[2];
+#pragma unroll
+    for (int a = 0; a < RA; ++a) x[a] = *reinterpret_cast<const f32x4_t*>(xs + xoff + 32 * a * kMRow + 8 * g);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) y[b] = *reinterpret_cast<const f32x4_t*>(ys + yoff + 32 * b * kMRow + 8 * g);
+#pragma unroll
+    for (int s = 0; s < decltype(steps)::value; ++s)
+#pragma unroll
+      for (int a = 0; a < RA; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = mfma_f32(x[a][s], y[b][s], acc[a][b]);
   };
   load_slice(0);
-  for (int e0 = 0; e0 < p.P; e0 += kGS) {
+  int e0 = 0;
+  for (; e0 + kMS <= p.P; e0 += kMS) {
     __syncthreads();  // the previous slice has been read
-#pragma unroll
-    for (int t = 0; t < kLoadsQ; ++t) {
-      const int idx = tid + 256 * t, blk = idx / kD4, d4 = idx % kD4;
-      float* x = xs + 4 * d4 * kXRow + blk;
-      x[0] = qv[t].x;
-      x[kXRow] = qv[t].y;
-      x[2 * kXRow] = qv[t].z;
-      x[3 * kXRow] = qv[t].w;
-    }
-#pragma unroll
-    for (int t = 0; t < kLoads; ++t) {
-      const int idx = tid + 256 * t, blk = idx / kD4, d4 = idx % kD4;
-#pragma unroll
-      for (int c = 0; c < PK; ++c) {
-        float* y = ys + (c * kGS + 4 * d4) * kYRow + blk;
-        y[0] = kv[c][t].x;
-        y[kYRow] = kv[c][t].y;
-        y[2 * kYRow] = kv[c][t].z;
-        y[3 * kYRow] = kv[c][t].w;
-      }
-    }
+    store_slice();
     __syncthreads();
-    if (e0 + kGS < p.P) load_slice(e0 + kGS);
-#pragma unroll 8
-    for (int e = 0; e < kGS; ++e) {
-      float x[TR];
+    if (e0 + kMS < p.P) load_slice(e0 + kMS);
+    if (live) {
 #pragma unroll
-      for (int r = 0; r < TR; r += 2) {
-        const float2 x2 = *reinterpret_cast<const float2*>(xs + e * kXRow + TR * tr + r);
-        x[r] = x2.x;
-        x[r + 1] = x2.y;
-      }
-#pragma unroll
-      for (int c = 0; c < PK; ++c) {
-        const float4 y4 = *reinterpret_cast<const float4*>(ys + (c * kGS + e) * kYRow + 4 * tc);
-        const float y[4] = {y4.x, y4.y, y4.z, y4.w};
-#pragma unroll
-        for (int r = 0; r < TR; ++r)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) acc[c][r][k] = __builtin_fmaf(x[r], y[k], acc[c][r][k]);
-      }
+      for (int g = 0; g < kMS / 8; ++g) group(g, std::integral_constant<int, 4>{});
     }
   }
-#pragma unroll
-  for (int r = 0; r < TR; ++r) {
-    const int i = i0 + TR * tr + r;
-    if (i >= p.Qb) continue;
-    float v[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int j = j0 + 4 * tc + k;
-      float best = acc[0][r][k];
-#pragma unroll
-      for (int c = 1; c < PK; ++c) best = acc[c][r][k] > best ? acc[c][r][k] : best;
-      v[k] = (!p.causal || j <= i) ? best / p.div : -INFINITY;
-    }
-    float* o = out + (int64_t)i * p.Kb + j0 + 4 * tc;
-    if (j0 + 4 * tc + 3 < p.Kb && (p.Kb & 3) == 0) {
-      *reinterpret_cast<float4*>(o) = float4{v[0], v[1], v[2], v[3]};
-    } else {
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (j0 + 4 * tc + k < p.Kb) o[k] = v[k];
+  if (e0 < p.P) {
+    __syncthreads();
+    store_slice();
+    __syncthreads();
+    if (live) {
+      for (int g = 0; g < (p.P - e0) / 8; ++g) group(g, std::integral_constant<int, 4>{});
+      if ((p.P - e0) % 8) group((p.P - e0) / 8, std::integral_constant<int, 2>{});
     }
   }
+  if (!live) {
+    // Above the diagonal inside a computed tile (or outside the matrix).
+    if (p.causal == 1)
+      for (int e = lane; e < (32 * RA / PQ) * (64 / PK); e += 64) {
+        const int i = iw + e / (64 / PK), j = jw + e % (64 / PK);
+        if (i < p.Qb && j < p.Kb) out[(int64_t)i * p.Kb + j] = -INFINITY;
+      }
+    return;
+  }
+  constexpr int GS = PQ < 4 ? PQ : 4;  // rows of one query block among a lane's four consecutive ones
+#pragma unroll
+  for (int a = 0; a < RA; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r0 = 0; r0 < 16; r0 += GS) {
+        const float first = acc[a][b][r0];
+        float m = first;
+#pragma unroll
+        for (int r = 1; r < GS; ++r) m = fmaxf(m, acc[a][b][r0 + r]);
+        if constexpr (PQ == 8) m = half_max(m);
+        if constexpr (PK >= 2) m = dpp_max<0xB1>(m);   // quad_perm [1, 0, 3, 2]
+        if constexpr (PK >= 4) m = dpp_max<0x4E>(m);   // quad_perm [2, 3, 0, 1]
+        if constexpr (PK >= 8) m = dpp_max<0x141>(m);  // row_half_mirror
+        if (first != first) m = first;
+        const int row = 32 * a + 8 * (r0 / 4) + (PQ == 8 ? 0 : 4 * (lane >> 5)) + r0 % 4;
+        const int i = iw + row / PQ, j = jw + (32 * b + (lane & 31)) / PK;
+        if (lane % PK == 0 && (PQ < 8 || lane < 32) && i < p.Qb && j < p.Kb)
+          out[(int64_t)i * p.Kb + j] = (!p.causal || j <= i) ? m / p.div : -INFINITY;
+      }
 }
 
 // The same scores for prototype counts whose tiles do not fit in LDS (e.g.
@@ -1833,15 +1917,9 @@ extern "C" int spruce_gate_project(const float* x, const float* w, int64_t N, in
   SPRUCE_REQUIRE(N >= 1 && D >= 1 && P >= 1 && N * P < ((int64_t)1 << 40), "invalid projection shape");
   const bool vec = D % 4 == 0 && P % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0 &&
                    ((uintptr_t)out % 16) == 0;
-  if (vec && N >= kBlockProjectRows) {
-    constexpr int TR = kBlockProjectTR, TC = kBlockProjectTC;
-    const int64_t brows = (N + 16 * TR - 1) / (16 * TR);
-    SPRUCE_REQUIRE(brows < ((int64_t)1 << 31) && P < ((int64_t)1 << 20) && D < ((int64_t)1 << 20),
-                   "projection too large");
-    hipLaunchKernelGGL((project_block_kernel<TR, TC, ProjRowsF32>),
-                       dim3((unsigned)brows, (unsigned)((P + 16 * TC - 1) / (16 * TC))), dim3(256), 0,
-                       (hipStream_t)stream, ProjRowsF32{x}, w, N, (int)D, (int)P, out);
-    return check_launch("project_block_kernel");
+  if (vec && N >= kMfmaProjectRows) {
+    SPRUCE_REQUIRE(P < ((int64_t)1 << 20) && D < ((int64_t)1 << 20), "projection too large");
+    return launch_project_mfma(ProjRowsF32{x}, w, 1, N, (int)D, (int)P, out, false, 0, (hipStream_t)stream);
   }
   if (vec) {
     const int64_t vrows = (N + 63) / 64;
@@ -1860,9 +1938,9 @@ extern "C" int spruce_gate_project(const float* x, const float* w, int64_t N, in
   return check_launch("project_kernel");
 }
 
-extern "C" int spruce_gate_project_levels(const void* const* levels, const int64_t* level_nodes, int64_t nlevels,
-                                          int64_t S, int64_t Pk, int64_t D, int dtype, const float* w, int64_t P,
-                                          float* out, int layout, void* stream) {
+extern "C" int spruce_gate_project_layers(const void* const* levels, const int64_t* level_nodes, int64_t nlevels,
+                                          int64_t L, int64_t S, int64_t Pk, int64_t D, int dtype, const float* w,
+                                          int64_t P, float* out, int layout, void* stream) {
   SPRUCE_REQUIRE(levels && level_nodes && w && out, "levels, level_nodes, w and out must be non-null");
   SPRUCE_REQUIRE(layout == SPRUCE_KP_ROWS || layout == SPRUCE_KP_INTERLEAVED, "unknown output layout %d", layout);
   SPRUCE_REQUIRE(nlevels >= 1 && nlevels <= kProjMaxSeg, "between 1 and %d levels, got %lld", kProjMaxSeg,
@@ -1889,29 +1967,21 @@ extern "C" int spruce_gate_project_levels(const void* const* levels, const int64
   g.off[nlevels] = total;
   g.N = total;
   const int64_t N = S * total * Pk;
-  SPRUCE_REQUIRE(N * P < ((int64_t)1 << 40), "projection too large");
-  constexpr int TR = kBlockProjectTR, TC = kBlockProjectTC;
-  const int64_t brows = (N + 16 * TR - 1) / (16 * TR);
-  SPRUCE_REQUIRE(brows < ((int64_t)1 << 31), "projection too large");
-  const dim3 grid((unsigned)brows, (unsigned)((P + 16 * TC - 1) / (16 * TC)));
+  SPRUCE_REQUIRE(L >= 1 && L < 65536 && N * P < ((int64_t)1 << 40) && L * N * P < ((int64_t)1 << 40),
+                 "projection too large");
   const hipStream_t st = (hipStream_t)stream;
   const bool il = layout == SPRUCE_KP_INTERLEAVED;
-  auto go = [&](auto rows) {
-    using RowsT = decltype(rows);
-    if (il)
-      hipLaunchKernelGGL((project_block_kernel<TR, TC, RowsT, true>), grid, dim3(256), 0, st, rows, w, N, (int)D,
-                         (int)P, out, (int)Pk);
-    else
-      hipLaunchKernelGGL((project_block_kernel<TR, TC, RowsT, false>), grid, dim3(256), 0, st, rows, w, N, (int)D,
-                         (int)P, out, 0);
-  };
   if (dtype == SPRUCE_DTYPE_BF16)
-    go(ProjRowsSeg<InBF16>{g});
-  else if (dtype == SPRUCE_DTYPE_F16)
-    go(ProjRowsSeg<InF16>{g});
-  else
-    go(ProjRowsSeg<InF32>{g});
-  return check_launch("project_block_kernel");
+    return launch_project_mfma(ProjRowsSeg<InBF16>{g}, w, L, N, (int)D, (int)P, out, il, (int)Pk, st);
+  if (dtype == SPRUCE_DTYPE_F16)
+    return launch_project_mfma(ProjRowsSeg<InF16>{g}, w, L, N, (int)D, (int)P, out, il, (int)Pk, st);
+  return launch_project_mfma(ProjRowsSeg<InF32>{g}, w, L, N, (int)D, (int)P, out, il, (int)Pk, st);
+}
+
+extern "C" int spruce_gate_project_levels(const void* const* levels, const int64_t* level_nodes, int64_t nlevels,
+                                          int64_t S, int64_t Pk, int64_t D, int dtype, const float* w, int64_t P,
+                                          float* out, int layout, void* stream) {
+  return spruce_gate_project_layers(levels, level_nodes, nlevels, 1, S, Pk, D, dtype, w, P, out, layout, stream);
 }
 
 // Both selector projections in one launch (32-row tiles: at the selector's
@@ -1925,7 +1995,7 @@ extern "C" int spruce_gate_project2(const float* xa, const float* wa, int64_t Na
   auto aligned = [](const void* q) { return ((uintptr_t)q % 16) == 0; };
   const bool vec = D % 4 == 0 && P % 4 == 0 && aligned(xa) && aligned(wa) && aligned(outa) && aligned(xb) &&
                    aligned(wb) && aligned(outb);
-  if (!vec || Na >= kBlockProjectRows || Nb >= kBlockProjectRows) {
+  if (!vec || Na >= kMfmaProjectRows || Nb >= kMfmaProjectRows) {
     const int rc = spruce_gate_project(xa, wa, Na, D, P, outa, stream);
     return rc != 0 ? rc : spruce_gate_project(xb, wb, Nb, D, P, outb, stream);
   }
@@ -1949,6 +2019,48 @@ extern "C" int spruce_gate_scores(const float* qp, const float* kp, int64_t BG, 
                  "score shape out of range");
   SPRUCE_REQUIRE(causal >= 0 && causal <= 2, "causal must be 0, 1 or 2, got %d", causal);
   ScoreParams p{qp, kp, scores, (int)Qb, (int)Kb, (int)Pq, (int)Pk, (int)P, div, causal};
+  const bool tri = causal == 2 && Qb == Kb;
+  if (!tri && causal == 2) p.causal = 1;
+  auto pow2 = [](int64_t n) { return n == 1 || n == 2 || n == 4 || n == 8; };
+  if (pow2(Pq) && pow2(Pk)) {
+    const int64_t ntj = (Kb * Pk + 127) / 128;
+    // Tiles of one slab at row tiles of TM prototype rows: with a square
+    // causal matrix only the tiles that reach the diagonal.
+    auto slab = [&](int64_t TM) {
+      const int64_t nti = (Qb * Pq + TM - 1) / TM, TI = TM / Pq, TJ = 128 / Pk;
+      if (!causal || Qb != Kb) return nti * ntj;
+      const int64_t q = TI >= TJ ? TI / TJ : 1, b = TI >= TJ ? 1 : TJ / TI, a = nti / b, r = nti - a * b;
+      return q * (b * (a * (a + 1) / 2) + r * (a + 1));
+    };
+    SPRUCE_REQUIRE((Qb * Pq + 63) / 64 * ntj < ((int64_t)1 << 31), "score matrix too large");
+    // 128-row tiles once they give every CU two workgroups; smaller grids take 64-row tiles.
+    const bool big = BG * slab(128) >= 512;
+    const int64_t nti = (Qb * Pq + (big ? 127 : 63)) / (big ? 128 : 64);
+    const int64_t per_slab = slab(big ? 128 : 64), tiles = BG * per_slab, per = (tiles + 7) / 8;
+    SPRUCE_REQUIRE(8 * per < ((int64_t)1 << 31), "score matrix too large");
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * per)), dim3(256), 0, (hipStream_t)stream, p, (int)nti, (int)ntj,
+                         per_slab, tiles, per);
+    };
+    auto pick = [&](auto pq, auto pk) {
+      constexpr int A = decltype(pq)::value, C = decltype(pk)::value;
+      if (big)
+        go(gate_scores_mfma_kernel<A, C, 2>);
+      else
+        go(gate_scores_mfma_kernel<A, C, 1>);
+    };
+    auto pick_k = [&](auto pq) {
+      if (Pk == 1) pick(pq, std::integral_constant<int, 1>{});
+      else if (Pk == 2) pick(pq, std::integral_constant<int, 2>{});
+      else if (Pk == 4) pick(pq, std::integral_constant<int, 4>{});
+      else pick(pq, std::integral_constant<int, 8>{});
+    };
+    if (Pq == 1) pick_k(std::integral_constant<int, 1>{});
+    else if (Pq == 2) pick_k(std::integral_constant<int, 2>{});
+    else if (Pq == 4) pick_k(std::integral_constant<int, 4>{});
+    else pick_k(std::integral_constant<int, 8>{});
+    return check_launch("gate_scores_mfma_kernel");
+  }
   const int64_t lds = (int64_t)(kTI * Pq * P + kTJ * (Pk * P + 4)) * 4;
   if (lds > 160 * 1024) {
     const int64_t total = BG * Qb * Kb;
@@ -1957,23 +2069,6 @@ extern "C" int spruce_gate_scores(const float* qp, const float* kp, int64_t BG, 
     hipLaunchKernelGGL(gate_scores_direct_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, p,
                        total);
     return check_launch("gate_scores_direct_kernel");
-  }
-  const bool tri = causal == 2 && Qb == Kb;
-  if (!tri && causal == 2) p.causal = 1;
-  if (Pq == 1 && (Pk == 1 || Pk == 2) && P % kGS == 0 && reinterpret_cast<uintptr_t>(scores) % 16 == 0) {
-    // 32-query-block tiles: twice as many workgroups as 64-block tiles,
-    // which evens out the per-CU share of a few hundred tiles.
-    constexpr int TR = kScoreTR, R = 16 * TR;
-    const int64_t nt = (Qb + kGT - 1) / kGT;
-    const int64_t ntri = (kGT / R) * (nt * (nt + 1) / 2);
-    SPRUCE_REQUIRE(!tri || BG * ntri < ((int64_t)1 << 31), "score matrix too large");
-    const dim3 grid = tri ? dim3((unsigned)(BG * ntri))
-                          : dim3((unsigned)((Qb + R - 1) / R), (unsigned)((Kb + kGT - 1) / kGT), (unsigned)BG);
-    if (Pk == 1)
-      hipLaunchKernelGGL((gate_scores_tile_kernel<1, TR>), grid, dim3(256), 0, (hipStream_t)stream, p);
-    else
-      hipLaunchKernelGGL((gate_scores_tile_kernel<2, TR>), grid, dim3(256), 0, (hipStream_t)stream, p);
-    return check_launch("gate_scores_tile_kernel");
   }
   const dim3 grid((unsigned)((Qb + kTI - 1) / kTI), (unsigned)((Kb + kTJ - 1) / kTJ), (unsigned)BG);
   if (lds > 64 * 1024) {

@@ -16,7 +16,7 @@ import torch
 import torch.nn as nn
 
 import spruce_hip
-from selector.select import gate_scores, project, project_levels
+from selector.select import gate_scores, project, project_layers
 
 
 class FlatGate(nn.Module):
@@ -38,14 +38,15 @@ class FlatGate(nn.Module):
     def _project(feat, W):
         """``[L, ..., d] -> [L, ..., p]`` float32; 16-bit features are read as they
         are (widened exactly in the kernel), float32 ones directly."""
-        def one(x, w):
-            if x.dtype in (torch.bfloat16, torch.float16) and x.shape[-1] % 4 == 0 and w.shape[-1] % 4 == 0:
-                rows = x.reshape(1, -1, 1, x.shape[-1])
-                return project_levels([rows], w).reshape(x.shape[:-1] + (w.shape[-1],))
-            return project(x.float(), w.float())
-        if feat.shape[0] == 1:
-            return one(feat[0], W[0]).unsqueeze(0)
-        return torch.stack([one(feat[l], W[l]) for l in range(feat.shape[0])])
+        L, (d, p) = feat.shape[0], W.shape[1:]
+        if 1 <= L <= W.shape[0] and feat.shape[-1] == d and d % 4 == 0 and p % 4 == 0 and feat.numel() and \
+                feat.dtype in (torch.bfloat16, torch.float16, torch.float32):
+            rows = feat.reshape(L, 1, -1, 1, d).contiguous()
+            if rows.data_ptr() % 16 == 0:   # every layer in one launch
+                return project_layers([rows], W[:L]).reshape(feat.shape[:-1] + (p,))
+        if L == 1:
+            return project(feat[0].float(), W[0].float()).unsqueeze(0)
+        return torch.stack([project(feat[l].float(), W[l].float()) for l in range(L)])
 
     @torch.no_grad()
     def project_key_levels(self, level_features, interleaved=False):
@@ -61,11 +62,7 @@ class FlatGate(nn.Module):
             if interleaved:
                 out = out.reshape(out.shape[:4] + (self.proj_dim // 4, 4)).transpose(3, 4).contiguous()
             return out
-        outs = []
-        for l in range(L):
-            outs.append(project_levels([f[l] for f in level_features], self.Wk[l], interleaved=interleaved))
-        out = outs[0].unsqueeze(0) if L == 1 else torch.stack(outs)
-        return out
+        return project_layers(level_features, self.Wk[:L], interleaved=interleaved)
 
     @torch.no_grad()
     def project_queries(self, q_feat):

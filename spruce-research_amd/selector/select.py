@@ -146,30 +146,42 @@ def project_levels(levels, W, interleaved=False):
     the tree traversal reads fastest."""
     if not levels:
         raise ValueError("levels must not be empty")
+    if W.dim() != 2 or W.shape[0] != levels[0].shape[-1]:
+        raise ValueError(f"shape mismatch: levels [..., {levels[0].shape[-1]}] @ W {tuple(W.shape)}")
+    return project_layers([t.unsqueeze(0) for t in levels], W.unsqueeze(0), interleaved=interleaved)[0]
+
+
+def project_layers(levels, W, interleaved=False):
+    """``project_levels`` of L layers in one launch: ``levels`` holds
+    ``[L, S, n_v, P, D]`` tensors and ``W`` is ``[L, D, p]``, one weight per
+    layer.  Returns ``[L, S, sum n_v, P, p]`` (or its interleaved form), the
+    values of L ``project_levels`` calls."""
+    if not levels:
+        raise ValueError("levels must not be empty")
     for t in levels:
         _cuda(t, "levels")
-    S, _, P, D = levels[0].shape
+    L, S, _, P, D = levels[0].shape
     dtype = levels[0].dtype
     for t in levels:
-        if t.dim() != 4 or t.shape[0] != S or t.shape[2:] != (P, D) or t.dtype != dtype:
+        if t.dim() != 5 or t.shape[:2] != (L, S) or t.shape[3:] != (P, D) or t.dtype != dtype:
             raise ValueError("levels must be [S, n, P, D] with one S, P, D and dtype")
-    if W.dim() != 2 or W.shape[0] != D:
-        raise ValueError(f"shape mismatch: levels [..., {D}] @ W {tuple(W.shape)}")
+    if W.dim() != 3 or W.shape[:2] != (L, D):
+        raise ValueError(f"shape mismatch: levels [..., {D}] of {L} layers @ W {tuple(W.shape)}")
     W = W.to(device=levels[0].device, dtype=torch.float32).contiguous()
     bufs = [t.contiguous() for t in levels]
-    nodes = [t.shape[1] for t in bufs]
-    p = W.shape[1]
+    nodes = [t.shape[2] for t in bufs]
+    p = W.shape[2]
     if interleaved and p % 4:
         raise ValueError("the interleaved layout needs a projection dim divisible by 4")
-    shape = (S, sum(nodes), p // 4, P, 4) if interleaved else (S, sum(nodes), P, p)
+    shape = (L, S, sum(nodes), p // 4, P, 4) if interleaved else (L, S, sum(nodes), P, p)
     out = torch.empty(shape, device=bufs[0].device, dtype=torch.float32)
     ptrs = (ctypes.c_void_p * len(bufs))(*[t.data_ptr() for t in bufs])
     counts = (ctypes.c_int64 * len(bufs))(*nodes)
     with torch.cuda.device(bufs[0].device):
-        rc = spruce_hip.lib().spruce_gate_project_levels(
-            ptrs, counts, len(bufs), S, P, D, spruce_hip.dtype_code(bufs[0]), spruce_hip.ptr(W), W.shape[1],
+        rc = spruce_hip.lib().spruce_gate_project_layers(
+            ptrs, counts, len(bufs), L, S, P, D, spruce_hip.dtype_code(bufs[0]), spruce_hip.ptr(W), p,
             spruce_hip.ptr(out), 1 if interleaved else 0, spruce_hip.stream_of(bufs[0]))
-    spruce_hip.check(rc, "spruce_gate_project_levels")
+    spruce_hip.check(rc, "spruce_gate_project_layers")
     return out
 
 

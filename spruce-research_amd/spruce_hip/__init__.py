@@ -53,6 +53,8 @@ _SIGNATURES = {
     "spruce_gate_project2": [_p, _p, _i64, _p, _p, _i64, _i64, _i64, _p, _p, _p],
     "spruce_gate_project_levels": [ctypes.POINTER(_p), _STRIDES, _i64, _i64, _i64, _i64, ctypes.c_int, _p, _i64,
                                    _p, ctypes.c_int, _p],
+    "spruce_gate_project_layers": [ctypes.POINTER(_p), _STRIDES, _i64, _i64, _i64, _i64, _i64, ctypes.c_int, _p, _i64,
+                                   _p, ctypes.c_int, _p],
     "spruce_gate_scores": [_p, _p, _i64, _i64, _i64, _i64, _i64, _i64, ctypes.c_float, ctypes.c_int, _p, _p],
     "spruce_causal_topk": [_p, _i64, _i64, _i64, _i64, _p, _p],
     "spruce_select_flat_supported": [_i64, _i64, _i64, _i64, ctypes.c_int, _i64],

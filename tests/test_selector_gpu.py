@@ -403,3 +403,54 @@ def test_pool_project_equals_pool_then_project(B, Hq, Hkv, T, dtype, bthd):
         exp = osel.flat_select(q.float().cpu().numpy(), kk.float().cpu().numpy(), Wq.cpu().numpy(),
                                Wk.cpu().numpy(), top_k=8)
         assert np.array_equal(_np(select_blocks(q, kk, Wq, Wk, top_k=8)), exp["selected"])
+
+
+@pytest.mark.parametrize("Pq", [1, 2, 4, 8])
+@pytest.mark.parametrize("Pk", [1, 2, 4, 8])
+def test_matrix_scores_are_bit_exact(Pq, Pk):
+    # The matrix-core scores over tile remainders, the projection dim's slices
+    # (32) and their tails, both tile heights and every causal form, against
+    # the oracle; NaN and infinities follow "replace when strictly larger".
+    gen = torch.Generator().manual_seed(10 * Pq + Pk)
+    for S, Qb, Kb, P in ((1, 1, 1, 4), (2, 33, 33, 36), (1, 70, 131, 64), (3, 129, 65, 32),
+                         (64, 512 // Pq, 512 // Pk, 4)):
+        qp = torch.randn(S, Qb, Pq, P, generator=gen)
+        kp = torch.randn(S, Kb, Pk, P, generator=gen)
+        if P == 36:
+            qp[0, 3, 0, 1], qp[0, 5, -1, 35], kp[1, 7, 0, 2], kp[1, 9, -1, 33] = (float("nan"), float("inf"),
+                                                                                 float("nan"), float("-inf"))
+        print(f"scores Pq={Pq} Pk={Pk} S={S} Qb={Qb} Kb={Kb} P={P}", flush=True)
+        for causal in (False, True) + (("lower",) if Qb == Kb else ()):
+            got = _np(gate_scores(qp.to(DEV), kp.to(DEV), causal=causal))
+            want = osel.scores(qp.numpy(), kp.numpy(), causal=bool(causal))
+            if causal == "lower":
+                low = np.tril(np.ones((Qb, Kb), bool))
+                got, want = got[:, low], want[:, low]
+            np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("L,S,nodes,Pk,D,P", [
+    (1, 1, [1], 1, 4, 4), (3, 2, [37, 19, 1], 8, 36, 64), (2, 1, [70], 4, 128, 132), (2, 3, [1500, 750, 5], 8, 32, 260)])
+def test_projection_of_layers_equals_each_layer(dtype, L, S, nodes, Pk, D, P):
+    # One launch over layers and levels (both tile heights, row and column
+    # remainders, tails of the 32-wide slices, both output layouts) against
+    # the small-row projection of each layer's float32 copy.
+    from selector.select import project_layers
+    gen = torch.Generator().manual_seed(sum(nodes) + D)
+    levels = [torch.randn(L, S, n, Pk, D, generator=gen).to(dtype).to(DEV) for n in nodes]
+    W = torch.randn(L, D, P, generator=gen).to(DEV)
+    print(f"project_layers {dtype} L={L} S={S} nodes={nodes} D={D} P={P}", flush=True)
+    x = torch.cat(levels, dim=2).float().reshape(L, -1, D)
+    want = torch.stack([torch.cat([project(c, W[l]) for c in x[l].split(8192)]) for l in range(L)])
+    want = want.reshape(L, S, sum(nodes), Pk, P)
+    assert torch.equal(project_layers(levels, W), want)
+    il = project_layers(levels, W, interleaved=True)
+    assert torch.equal(il.transpose(3, 4).reshape(want.shape), want)
+    if len(nodes) == 1:
+        gate = FlatGate(L + 1, D, proj_dim=P).to(DEV)
+        with torch.no_grad():
+            gate.Wq[:L].copy_(W)
+        assert torch.equal(gate.project_queries(levels[0]), want)
+        odd = torch.empty(levels[0].numel() + 1, dtype=dtype, device=DEV)[1:].view(levels[0].shape).copy_(levels[0])
+        assert torch.equal(gate.project_queries(odd), want)   # not 16-byte aligned: the general kernels
