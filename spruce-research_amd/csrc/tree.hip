@@ -28,6 +28,8 @@
 //           candidates with the largest score, ties to the lower node index,
 //           score-descending; missing slots are -1 (the reference ranks
 //           invalid candidates at finfo.min after every valid one).
+#include <utility>
+
 #include "common.h"
 
 namespace spruce {
@@ -349,6 +351,116 @@ __device__ __forceinline__ void maxsim_multi(const float* qrow, const float* con
   }
 }
 
+// The same chains on the matrix cores, for 4 or 8 query prototypes and p = 64
+// or 128.  v_mfma_f32_4x4x1_16b_f32 is 16 products of 4 rows x 4 columns, one
+// multiply-add per element with a single rounding, so a sequence of them over
+// e is the fmaf chain bit for bit (compared on the GPU over normal,
+// wide-exponent, denormal and special operands).  Column l % 4 of block l / 4
+// is lane l's key vector, so lane l receives its pair's products with four
+// query prototypes, and with cbsz = 4 every block takes the rows of block
+// `abid`: one register of the query operand holds 16 dims, one per block, so
+// 16 dims of four queries are one LDS read.  4 x 2048 rows, 2048 leaves, 8 x 8
+// prototypes, beam 16: 560 us (VALU chains) -> 372 us.  What bounds it now are
+// the key vectors, 6.6 GB through the 64 bytes a clock of each CU's vector
+// cache (about 230 us alone), and the products (120 TFLOP/s on random values,
+// 215 us alone), of which a SIMD's few waves overlap about a half.
+template <int PQ, int NP, int J, int E>
+__device__ __forceinline__ void mfma_dims(const float (&q)[PQ / 4], const f32x4_t (&k)[NP][4],
+                                          f32x4_t (&acc)[NP][PQ / 4]) {
+#pragma unroll
+  for (int n = 0; n < NP; ++n)
+#pragma unroll
+    for (int h = 0; h < PQ / 4; ++h)
+      acc[n][h] = __builtin_amdgcn_mfma_f32_4x4x1f32(q[h], k[n][J][E], acc[n][h], 4, 4 * J + E, 0);
+#pragma unroll
+  for (int n = 0; n < NP; ++n)
+#pragma unroll
+    for (int h = 0; h < PQ / 4; ++h)
+      acc[n][h] = __builtin_amdgcn_mfma_f32_4x4x1f32(q[h], k[n][J][E + 1], acc[n][h], 4, 4 * J + E + 1, 0);
+}
+
+// qf: the query operand in LDS, [PQ / 4][PD / 16][64 lanes].  A wave issues in
+// order and a load takes the address unit about 16 cycles, so a piece's loads
+// go one at a time between the products of the piece before it (in a burst
+// they hold up the products: 476 against 386 us).
+template <int PQ, int PD, int NP, int GS>
+__device__ __forceinline__ void maxsim_mfma(const float* qf, const float* const (&kv)[NP], int gs_rt, int lane,
+                                            float (&res)[NP]) {
+  const int gs = GS > 0 ? GS : gs_rt;
+  constexpr int H = PQ / 4, R = PD / 16;
+  f32x4_t acc[NP][H], ka[NP][4], kb[NP][4];
+  float qa[H], qb[H];
+#pragma unroll
+  for (int n = 0; n < NP; ++n)
+#pragma unroll
+    for (int h = 0; h < H; ++h) acc[n][h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int n = 0; n < NP; ++n) ka[n][j] = *reinterpret_cast<const f32x4_t*>(kv[n] + (int64_t)j * gs);
+#pragma unroll
+  for (int h = 0; h < H; ++h) qa[h] = qf[h * R * 64 + lane];
+  // One piece's products; with `more` the loads of piece `next` go between them.
+  auto piece = [&](auto more, int next, const f32x4_t (&k)[NP][4], const float (&q)[H], f32x4_t (&kn)[NP][4],
+                   float (&qn)[H]) {
+    constexpr bool kNext = decltype(more)::value;
+    if constexpr (kNext) {
+#pragma unroll
+      for (int h = 0; h < H; ++h) qn[h] = qf[(h * R + next) * 64 + lane];
+    }
+    auto quad = [&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      auto half = [&](auto hc) {
+        constexpr int i = decltype(hc)::value;  // dims 2 i, 2 i + 1 of the quad
+        if constexpr (kNext && i < NP) {
+          kn[i][j] = *reinterpret_cast<const f32x4_t*>(kv[i] + (int64_t)(4 * next + j) * gs);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        mfma_dims<PQ, NP, j, 2 * i>(q, k, acc);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      half(std::integral_constant<int, 0>{});
+      half(std::integral_constant<int, 1>{});
+    };
+    quad(std::integral_constant<int, 0>{});
+    quad(std::integral_constant<int, 1>{});
+    quad(std::integral_constant<int, 2>{});
+    quad(std::integral_constant<int, 3>{});
+  };
+#pragma unroll 1
+  for (int r = 0; r + 2 < R; r += 2) {
+    piece(std::true_type{}, r + 1, ka, qa, kb, qb);
+    piece(std::true_type{}, r + 2, kb, qb, ka, qa);
+  }
+  piece(std::true_type{}, R - 1, ka, qa, kb, qb);
+  piece(std::false_type{}, 0, kb, qb, ka, qa);
+#pragma unroll
+  for (int n = 0; n < NP; ++n) {
+    // "Replace when strictly larger": NaN only from the first value, which
+    // fmaxf would drop.  (A maximum of zero may take either sign; scores
+    // order -0 and +0 as equal.)
+    const float x = acc[n][0][0];
+    float m = x;
+#pragma unroll
+    for (int a = 1; a < PQ; ++a) m = fmaxf(m, acc[n][a / 4][a % 4]);
+    res[n] = x != x ? x : m;
+  }
+}
+
+// The same maximum over the PK (4 or 8) lanes that hold a candidate's key
+// prototypes, valid in the first of them.
+template <int PK>
+__device__ __forceinline__ float max_over_prototypes(float x) {
+  auto step = [](float v, auto ctrl) {
+    return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v),
+                                                                      decltype(ctrl)::value, 0xf, 0xf, true)));
+  };
+  float m = step(x, std::integral_constant<int, 0xB1>{});   // quad_perm [1, 0, 3, 2]
+  m = step(m, std::integral_constant<int, 0x4E>{});         // quad_perm [2, 3, 0, 1]
+  if constexpr (PK == 8) m = step(m, std::integral_constant<int, 0x141>{});  // row_half_mirror
+  return x != x ? x : m;
+}
+
 // Two pairs per lane in 64-byte pieces.  Measured at the cfg5 grid against
 // 1.0-1.06 ms: four pairs in 64-byte pieces 1.68 ms (289 registers), four in
 // 32-byte pieces 1.10 ms, four or eight in 16-byte pieces 1.77-2.03 ms.
@@ -363,38 +475,53 @@ struct TraverseParams {
   int32_t* out;              // [S, qb, C]
 };
 
-// Scores pairs pr + 64 n (n < NP) of one level into pm.  An invalid or
-// missing pair reads the level's first node (always in range) and its result
-// is dropped.
-template <int PQ, int NP, int PD, int GS>
-__device__ __forceinline__ void score_pairs(const ScoreParams2& sc, const float* qrow, const float* kl,
-                                            const int* cand, const int* valid, int npairs, int lane,
-                                            float* pm) {
-  for (int pr = lane; pr < npairs; pr += 64 * NP) {
+// Scores pairs pr + 64 n (n < NP) of one level: pair = (candidate cand[i], key
+// prototype), the candidates all valid.  PK > 0: that many key prototypes, and
+// pm[i] takes candidate i's maximum over them; PK == 0: pm[pair].  A missing
+// pair reads the level's first node (always in range) and its result is
+// dropped.
+template <int NP, int PK, typename MaxSim>
+__device__ __forceinline__ void score_pairs(const ScoreParams2& sc, const float* kl, const int* cand, int nv, int lane,
+                                            float* pm, MaxSim maxsim) {
+  const int Pk = PK > 0 ? PK : sc.Pk, npairs = nv * Pk;
+  for (int p0 = 0; p0 < npairs; p0 += 64 * NP) {
+    const int pr = p0 + lane;
     int idx[NP], cc[NP];
-    bool ok[NP];
     const float* kv[NP];
 #pragma unroll
     for (int n = 0; n < NP; ++n) {
       const int pn = pr + 64 * n;
-      idx[n] = pn < npairs ? pn / sc.Pk : 0;
-      cc[n] = pn < npairs ? pn - idx[n] * sc.Pk : 0;
-      ok[n] = pn < npairs && valid[idx[n]] != 0;
-      kv[n] = kl + (ok[n] ? kvec(sc, cand[idx[n]], cc[n]) : 0);
+      idx[n] = pn < npairs ? pn / Pk : 0;
+      cc[n] = pn < npairs ? pn - idx[n] * Pk : 0;
+      kv[n] = kl + (pn < npairs ? (int64_t)cand[idx[n]] * Pk * sc.pd + (int64_t)cc[n] * sc.cstride : 0);
     }
     float m[NP];
-    maxsim_multi<PQ, NP, kTravCW, PD, GS>(qrow, kv, sc.pd, sc.gs, m);
+    maxsim(kv, m);
 #pragma unroll
-    for (int n = 0; n < NP; ++n)
-      if (pr + 64 * n < npairs) pm[idx[n] * sc.Pk + cc[n]] = ok[n] ? m[n] : 0.f;
+    for (int n = 0; n < NP; ++n) {
+      if constexpr (PK > 0) {
+        const float x = max_over_prototypes<PK>(m[n]);
+        if (pr + 64 * n < npairs && cc[n] == 0) pm[idx[n]] = x;
+      } else {
+        if (pr + 64 * n < npairs) pm[idx[n] * Pk + cc[n]] = m[n];
+      }
+    }
   }
 }
 
 // One wavefront per (slab, query block) row.  PQ > 0: that many query
 // prototypes, two pairs per lane per step (one on levels of at most 64
-// pairs); PQ == 0: any count, one pair.
+// pairs), on the matrix cores for PQ = 4 or 8 with PD fixed; PQ == 0: any
+// count, one pair.
+//
+// A level's valid candidates are compacted before they are scored, and when
+// all of them enter the next beam (the levels near the root, and early query
+// blocks) they are not scored at all: above the leaves only the set matters.
+// At 2048 leaves and beam 16 that leaves 224 of 254 scored candidates a row.
 template <int PQ, int PD = 0, int GS = 0>
-__global__ __launch_bounds__(64) void tree_traverse_kernel(const TraverseParams p) {
+__global__ __launch_bounds__(64, PD > 0 ? 4 : 1) void tree_traverse_kernel(const TraverseParams p) {
+  constexpr bool kMfma = PD > 0 && PQ % 4 == 0 && PQ > 0;
+  constexpr int PK = kMfma && GS > 4 ? GS / 4 : 0;  // key prototypes, where the group stride tells them
   extern __shared__ float sh[];
   const ScoreParams2& sc = p.sc;
   const int64_t row = blockIdx.x;
@@ -402,66 +529,114 @@ __global__ __launch_bounds__(64) void tree_traverse_kernel(const TraverseParams 
   const int q = (int)(row - s * sc.qb);
   if (s >= sc.S) return;
   const int lane = threadIdx.x;
-  float* qrow = sh;                          // [Pq, p]
-  float* pm = qrow + sc.Pq * sc.pd;          // [64, Pk] per-(candidate, key prototype) max
-  int* cand = reinterpret_cast<int*>(pm + 64 * sc.Pk);   // [64]
-  int* valid = cand + 64;                    // [64]
-  int* sel = valid + 64;                     // [64] current beam (node index within level)
+  uint64_t* keys = reinterpret_cast<uint64_t*>(sh);      // [64] rank keys
+  float* qrow = sh + 128;                                // the queries, Pq * p floats
+  float* pm = qrow + sc.Pq * sc.pd;                      // [64, Pk] per-(candidate, key prototype) max
+  int* cand = reinterpret_cast<int*>(pm + 64 * (PK > 0 ? 1 : sc.Pk));  // [64] valid candidates
+  int* sel = cand + 64;                      // [64] current beam (node index within level)
   const float* qsrc = sc.qp + (s * sc.qb + q) * (int64_t)sc.Pq * sc.pd;
-  for (int i = lane; i < sc.Pq * sc.pd; i += 64) qrow[i] = qsrc[i];
+  if constexpr (kMfma) {
+#pragma unroll
+    for (int h = 0; h < PQ / 4; ++h)
+#pragma unroll
+      for (int r = 0; r < PD / 16; ++r)
+        qrow[(h * (PD / 16) + r) * 64 + lane] = qsrc[(4 * h + (lane & 3)) * PD + 16 * r + (lane >> 2)];
+  } else {
+    for (int i = lane; i < sc.Pq * sc.pd; i += 64) qrow[i] = qsrc[i];
+  }
   if (lane == 0) sel[0] = 0;  // the root
   int W = 1;
   __syncthreads();
   for (int v = p.levels - 2; v >= 0; --v) {
     const int ncand = W * p.radix;
+    int c = -1;
+    bool ok = false;
     if (lane < ncand) {
       const int par = sel[lane / p.radix];
-      const int c = par >= 0 ? par * p.radix + lane % p.radix : -1;
-      const bool ok = par >= 0 && c < p.count[v] && (int64_t)c * p.span[v] <= q;
-      cand[lane] = c;
-      valid[lane] = ok ? 1 : 0;
-    }
-    __syncthreads();
-    const float* kl = sc.kp + (s * sc.N + p.offset[v]) * (int64_t)sc.Pk * sc.pd;
-    const int npairs = ncand * sc.Pk;
-    if (PQ > 0 && sc.pd % (8 * kTravCW) == 0) {
-      // A level with at most 64 pairs (the tree's top levels) takes one pair
-      // per lane: with two, half of every lane's chains would be dropped.
-      if (npairs <= 64)
-        score_pairs<PQ == 0 ? 1 : PQ, 1, PD, GS>(sc, qrow, kl, cand, valid, npairs, lane, pm);
-      else
-        score_pairs<PQ == 0 ? 1 : PQ, kTravNP, PD, GS>(sc, qrow, kl, cand, valid, npairs, lane, pm);
-    } else {
-      for (int pr = lane; pr < npairs; pr += 64) {
-        const int i = pr / sc.Pk, c = pr - (pr / sc.Pk) * sc.Pk;
-        float m = 0.f;
-        if (valid[i]) m = maxsim_one(qrow, kl + kvec(sc, cand[i], c), sc.Pq, sc.pd, sc.gs);
-        pm[i * sc.Pk + c] = m;
-      }
-    }
-    __syncthreads();
-    // Each candidate's place in the order (valid first; then score
-    // descending, NaN first, equal scores to the lower node; invalid ones by
-    // lane) as one distinct 64-bit key, larger = earlier, so a rank is a
-    // count of larger keys: one 64-bit compare per other candidate.
-    uint64_t key = 0;
-    if (lane < ncand) {
-      float best = pm[lane * sc.Pk];
-      for (int c = 1; c < sc.Pk; ++c)
-        if (pm[lane * sc.Pk + c] > best) best = pm[lane * sc.Pk + c];
-      key = valid[lane] ? (1ull << 63) | ((uint64_t)score_order(best / sc.div) << 31) |
-                              (uint64_t)(0x7fffffff - cand[lane])
-                        : (uint64_t)(63 - lane);
+      c = par >= 0 ? par * p.radix + lane % p.radix : -1;
+      ok = par >= 0 && c < p.count[v] && (int64_t)c * p.span[v] <= q;
     }
     int k = p.beam < ncand ? p.beam : ncand;
     k = k < p.count[v] ? k : p.count[v];
-    int rank = 0;
-    for (int o = 0; o < ncand; ++o) {
-      const uint64_t ko = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(key >> 32), o) << 32) |
-                          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)key, o);
-      rank += ko > key ? 1 : 0;
+    const uint64_t okb = __ballot(ok);
+    const int nv = __popcll(okb);
+    const int pos = __popcll(okb & ((1ull << lane) - 1));
+    __syncthreads();  // sel has been read
+    if (v > 0 && nv <= k) {
+      // Every valid candidate enters the beam.
+      if (ok) sel[pos] = c;
+      if (lane >= nv && lane < k) sel[lane] = -1;
+      W = k;
+      __syncthreads();
+      continue;
     }
-    if (lane < ncand && rank < k) sel[rank] = valid[lane] ? cand[lane] : -1;
+    if (ok) cand[pos] = c;
+    __syncthreads();
+    const float* kl = sc.kp + (s * sc.N + p.offset[v]) * (int64_t)sc.Pk * sc.pd;
+    // A level with at most 64 pairs takes one pair per lane: with two, half
+    // of every lane's chains would be dropped.
+    const bool one = nv * (PK > 0 ? PK : sc.Pk) <= 64;
+    if constexpr (kMfma) {
+      if (one)
+        score_pairs<1, PK>(sc, kl, cand, nv, lane, pm, [&](const float* const (&kv)[1], float (&m)[1]) {
+          maxsim_mfma<PQ, PD, 1, GS>(qrow, kv, sc.gs, lane, m);
+        });
+      else
+        score_pairs<kTravNP, PK>(sc, kl, cand, nv, lane, pm,
+                                 [&](const float* const (&kv)[kTravNP], float (&m)[kTravNP]) {
+                                   maxsim_mfma<PQ, PD, kTravNP, GS>(qrow, kv, sc.gs, lane, m);
+                                 });
+    } else if (PQ > 0 && sc.pd % (8 * kTravCW) == 0) {
+      constexpr int Q = PQ == 0 ? 1 : PQ;
+      if (one)
+        score_pairs<1, 0>(sc, kl, cand, nv, lane, pm, [&](const float* const (&kv)[1], float (&m)[1]) {
+          maxsim_multi<Q, 1, kTravCW, PD, GS>(qrow, kv, sc.pd, sc.gs, m);
+        });
+      else
+        score_pairs<kTravNP, 0>(sc, kl, cand, nv, lane, pm,
+                                [&](const float* const (&kv)[kTravNP], float (&m)[kTravNP]) {
+                                  maxsim_multi<Q, kTravNP, kTravCW, PD, GS>(qrow, kv, sc.pd, sc.gs, m);
+                                });
+    } else {
+      for (int pr = lane; pr < nv * sc.Pk; pr += 64) {
+        const int i = pr / sc.Pk, c = pr - (pr / sc.Pk) * sc.Pk;
+        pm[i * sc.Pk + c] = maxsim_one(qrow, kl + kvec(sc, cand[i], c), sc.Pq, sc.pd, sc.gs);
+      }
+    }
+    __syncthreads();
+    // Each candidate's place in the order (score descending, NaN first, equal
+    // scores to the lower node) as one distinct 64-bit key, larger = earlier,
+    // so a rank is a count of larger keys.  Up to 32 candidates sit in both
+    // halves of the wave, each half counting over every second key.
+    uint64_t key = 0;
+    int mine = -1;
+    const int me = nv <= 32 ? lane & 31 : lane;
+    if (me < nv) {
+      mine = cand[me];
+      float best;
+      if constexpr (PK > 0) {
+        best = pm[me];
+      } else {
+        best = pm[me * sc.Pk];
+        for (int c = 1; c < sc.Pk; ++c)
+          if (pm[me * sc.Pk + c] > best) best = pm[me * sc.Pk + c];
+      }
+      key = ((uint64_t)score_order(best / sc.div) << 31) | (uint64_t)(0x7fffffff - mine);
+    }
+    keys[lane] = key;  // lanes past the last candidate: 0, below every key
+    __syncthreads();
+    int rank = 0;
+    if (nv <= 32) {
+      const int h = lane >> 5;
+#pragma unroll 8
+      for (int o = 0; o < nv; o += 2) rank += keys[o + h] > key ? 1 : 0;
+      rank += __shfl_xor(rank, 32);
+    } else {
+#pragma unroll 8
+      for (int o = 0; o < nv; ++o) rank += keys[o] > key ? 1 : 0;
+    }
+    if (lane < nv && rank < k) sel[rank] = mine;
+    if (lane >= nv && lane < k) sel[lane] = -1;
     W = k;
     __syncthreads();
   }
@@ -654,23 +829,33 @@ extern "C" int spruce_tree_traverse(const float* qp, const float* kp, int64_t S,
   p.levels = levels;
   p.C = (int)C;
   p.out = out;
-  const size_t lds = ((size_t)Pq * pd + 64 * Pk) * sizeof(float) + 3 * 64 * sizeof(int);
   const dim3 grid((unsigned)(S * qb));
-  switch (Pq) {
-    case 1: hipLaunchKernelGGL(tree_traverse_kernel<1>, grid, dim3(64), lds, (hipStream_t)stream, p); break;
-    case 2: hipLaunchKernelGGL(tree_traverse_kernel<2>, grid, dim3(64), lds, (hipStream_t)stream, p); break;
-    case 4: hipLaunchKernelGGL(tree_traverse_kernel<4>, grid, dim3(64), lds, (hipStream_t)stream, p); break;
-    case 8:
-      // The deployed shape (8 prototypes, p = 128) with compile-time strides.
-      if (pd == 128 && il && Pk == 8)
-        hipLaunchKernelGGL((tree_traverse_kernel<8, 128, 32>), grid, dim3(64), lds, (hipStream_t)stream, p);
-      else if (pd == 128 && !il)
-        hipLaunchKernelGGL((tree_traverse_kernel<8, 128, 4>), grid, dim3(64), lds, (hipStream_t)stream, p);
-      else
-        hipLaunchKernelGGL(tree_traverse_kernel<8>, grid, dim3(64), lds, (hipStream_t)stream, p);
-      break;
-    default: hipLaunchKernelGGL(tree_traverse_kernel<0>, grid, dim3(64), lds, (hipStream_t)stream, p); break;
-  }
+  const size_t lds =
+      64 * sizeof(uint64_t) + ((size_t)Pq * pd + 64 * Pk) * sizeof(float) + 2 * 64 * sizeof(int);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(64), lds, (hipStream_t)stream, p);
+  };
+  // Matrix-core scoring, with the key group stride fixed where it is known:
+  // as many key prototypes as query prototypes interleaved, or rows.
+  auto mfma = [&](auto pq, auto dim) {
+    constexpr int Q = decltype(pq)::value, D = decltype(dim)::value;
+    if (il && Pk == Q)
+      go(tree_traverse_kernel<Q, D, 4 * Q>);
+    else if (!il)
+      go(tree_traverse_kernel<Q, D, 4>);
+    else
+      go(tree_traverse_kernel<Q, D, 0>);
+  };
+  using std::integral_constant;
+  if (Pq == 8 && pd == 128) mfma(integral_constant<int, 8>{}, integral_constant<int, 128>{});
+  else if (Pq == 8 && pd == 64) mfma(integral_constant<int, 8>{}, integral_constant<int, 64>{});
+  else if (Pq == 4 && pd == 128) mfma(integral_constant<int, 4>{}, integral_constant<int, 128>{});
+  else if (Pq == 4 && pd == 64) mfma(integral_constant<int, 4>{}, integral_constant<int, 64>{});
+  else if (Pq == 8) go(tree_traverse_kernel<8>);
+  else if (Pq == 4) go(tree_traverse_kernel<4>);
+  else if (Pq == 2) go(tree_traverse_kernel<2>);
+  else if (Pq == 1) go(tree_traverse_kernel<1>);
+  else go(tree_traverse_kernel<0>);
   return check_launch("tree_traverse_kernel");
 }
 
