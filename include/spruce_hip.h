@@ -239,6 +239,19 @@ int spruce_sparse_prefill_index_amask(const void* q, const int64_t qs[4], const 
                                       const int64_t os[4], void* stream);
 
 /*
+ * Reduces a 4-D decoder mask [B, Hm, T, T] (element strides ms, last 1;
+ * mask_dtype as amask_dtype above) to per-token key validity: valid [B, T]
+ * uint8 is what the last query row attends, flags[0] is set unless the mask
+ * is causal key padding over it (the same for every head, 0 / <= finfo.min/2
+ * values, every row of a real token exactly its causal real keys, a padding
+ * row those, nothing or everything), and flags[1] is set when some key is
+ * padding.  flags must hold zeros.  Serves sparse_prefill_attention_forward's
+ * padded batches (sparse/attention.py:147-150,173-176 in the reference).
+ */
+int spruce_mask_key_validity(const void* mask, const int64_t ms[4], int64_t Hm, int mask_dtype, int64_t B, int64_t T,
+                             uint8_t* valid, int32_t* flags, void* stream);
+
+/*
  * Residual-tree frontiers.  Replaces build_residual_summary_nodes /
  * residual_frontier_for_row (interfaces/residual_summaries.py:119-222): for
  * each row (b, l, g, q) of selected [B, L, G, Qb, K] int32 (element strides

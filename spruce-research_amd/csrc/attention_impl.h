@@ -895,11 +895,16 @@ __global__ __launch_bounds__(WAVES * 64) void sparse_prefill_kernel(const AttnPa
     }
     if constexpr (KVAL) {
       // Register r of key tile c holds key 32c + 8(r/4) + 4(lane/32) + r%4.
+      // Most blocks of a padded prompt hold no padding: a scalar test spares
+      // them the 64 selects (4 x 2048 tokens, 32/8 heads, 12 blocks a row, a
+      // quarter of the tokens padding: 127.7 -> 122.3 us).
+      if (vb != ~0ull) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int kr = 8 * (r >> 2) + 4 * hl + (r & 3);
-        if (!((vb >> kr) & 1ull)) s0[r] = -INFINITY;
-        if (!((vb >> (32 + kr)) & 1ull)) s1[r] = -INFINITY;
+        for (int r = 0; r < 16; ++r) {
+          const int kr = 8 * (r >> 2) + 4 * hl + (r & 3);
+          if (!((vb >> kr) & 1ull)) s0[r] = -INFINITY;
+          if (!((vb >> (32 + kr)) & 1ull)) s1[r] = -INFINITY;
+        }
       }
     }
     if (diag) {

@@ -38,6 +38,7 @@ from typing import Optional
 
 import torch
 
+import spruce_hip
 from interfaces.residual_summaries import (build_residual_tree_layout,
                                           validate_residual_summary_nodes)
 from interfaces.validator import validate_selected_blocks
@@ -172,6 +173,29 @@ def _key_validity(attention_mask: torch.Tensor, batch: int, seq_len: int) -> Opt
     return valid
 
 
+_MASK_CODES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2, torch.bool: 3}
+
+
+def _key_validity_and_padding(attention_mask: torch.Tensor, batch: int, seq_len: int) -> tuple:
+    """(``_key_validity``, whether some key is padding) of a mask: on the GPU
+    one launch that reads the mask once and one read back of its two flags;
+    masks the kernel does not read (other dtypes, strided rows, host tensors)
+    take the tensor operations above."""
+    m = attention_mask
+    if not (m.is_cuda and m.dtype in _MASK_CODES and m.stride(-1) == 1 and m.numel()):
+        valid = _key_validity(m, batch, seq_len)
+        return valid, valid is not None and not bool(valid.all())
+    valid = torch.empty((batch, seq_len), device=m.device, dtype=torch.bool)
+    flags = torch.zeros(2, device=m.device, dtype=torch.int32)
+    with torch.cuda.device(m.device):
+        rc = spruce_hip.lib().spruce_mask_key_validity(
+            spruce_hip.ptr(m), spruce_hip.strides(m), m.shape[1], _MASK_CODES[m.dtype], batch, seq_len,
+            spruce_hip.ptr(valid), spruce_hip.ptr(flags), spruce_hip.stream_of(m))
+    spruce_hip.check(rc, "spruce_mask_key_validity")
+    other, padded = flags.tolist()
+    return (None, False) if other else (valid, bool(padded))
+
+
 def sparse_prefill_attention_forward(
     module: torch.nn.Module,
     query: torch.Tensor,
@@ -223,14 +247,14 @@ def sparse_prefill_attention_forward(
     general_mask = None
     if attention_mask is not None:
         _check_mask_shape(attention_mask, query.shape[0], query.shape[1], query.shape[-2])
-        key_valid = _key_validity(attention_mask, query.shape[0], query.shape[-2])
+        key_valid, padded = _key_validity_and_padding(attention_mask, query.shape[0], query.shape[-2])
         if key_valid is None:
             if residual_summaries:
                 raise ValueError(
                     "residual summaries on the HIP sparse-prefill path need a causal key-padding "
                     "attention mask; this mask has another pattern")
             general_mask = attention_mask   # added to the scores inside the kernel
-        elif bool(key_valid.all()):
+        elif not padded:
             key_valid = None      # no padding: the plain kernel
     if block_size != 64:
         raise ValueError("the HIP sparse-prefill kernel requires block_size=64")

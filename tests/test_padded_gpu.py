@@ -173,3 +173,65 @@ def test_padded_batch_through_a_qwen2_model():
           flush=True)
     assert torch.isfinite(sparse[real]).all()
     assert d.max().item() <= 2e-2 and d.mean().item() <= 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bool, torch.bfloat16, torch.float16, torch.float32])
+def test_mask_reduction_kernel_equals_the_tensor_operations(dtype):
+    # spruce_mask_key_validity against _key_validity over the forms it takes:
+    # padding on either side, opened and closed padding rows, other patterns,
+    # biases, NaN, per-head and expanded heads, sizes around the 16-byte and
+    # wave steps, unaligned and strided rows.
+    from sparse.attention import _key_validity, _key_validity_and_padding
+    gen = torch.Generator().manual_seed(5)
+    low = True if dtype == torch.bool else torch.finfo(dtype).min
+
+    def build(attend, fill=None):
+        if dtype == torch.bool:
+            return attend
+        return torch.zeros(attend.shape, dtype=dtype).masked_fill(~attend, low if fill is None else fill)
+
+    for T in (1, 2, 15, 16, 63, 64, 129, 1030):
+        B = 3
+        pos = torch.arange(T)
+        causal = pos[None, :] <= pos[:, None]
+        n = torch.randint(1, T + 1, (B,), generator=gen)
+        masks = [build((causal[None] & torch.ones(B, 1, T, dtype=torch.bool))[:, None])]
+        for left in (False, True):
+            valid = pos[None] >= T - n[:, None] if left else pos[None] < n[:, None]
+            att = causal[None] & valid[:, None, :]
+            masks.append(build(att[:, None]))
+            opened = att.clone()
+            opened[~valid] = True
+            masks.append(build(opened[:, None]))
+            closed = att.clone()
+            closed[~valid] = False
+            masks.append(build(closed[:, None]))
+            flip = att.clone()
+            flip[B - 1, T // 2, T // 3] ^= True
+            masks.append(build(flip[:, None]))
+            masks.append(build(att[:, None]).expand(B, 4, T, T))
+            heads = build(att[:, None].repeat(1, 3, 1, 1))
+            masks.append(heads)
+            other = heads.clone()
+            other[1, 2, T - 1, T // 2] = low if dtype == torch.bool and not other[1, 2, T - 1, T // 2] else (
+                False if dtype == torch.bool else 0.5)
+            masks.append(other)
+            if dtype != torch.bool:
+                for value in (-1.0, low / 2, float("-inf"), float("nan"), -0.0, 1.0):
+                    biased = build(att[:, None])
+                    biased[0, 0, T // 2, T - 1] = value
+                    masks.append(biased)
+                masks.append(build(att[:, None], float("-inf")))
+                masks.append(build(att[:, None], -1.0))
+        seg = (torch.rand(B, T, generator=gen) < 0.1).cumsum(-1)
+        masks.append(build((causal[None] & (seg[:, :, None] == seg[:, None, :]))[:, None]))
+        print(f"mask reduction {dtype} T={T}: {len(masks)} masks", flush=True)
+        for m in masks:
+            want = _key_validity(m, B, T)
+            wide = torch.empty(m.shape[:3] + (T + 3,), dtype=dtype)
+            wide[..., 3:] = m
+            for dev in (m.to(DEV), wide.to(DEV)[..., 3:], m.transpose(2, 3).contiguous().to(DEV).transpose(2, 3)):
+                got, padded = _key_validity_and_padding(dev, B, T)
+                assert (got is None) == (want is None)
+                if want is not None:
+                    assert torch.equal(got.cpu(), want) and padded == (not bool(want.all()))
