@@ -45,7 +45,7 @@ def selected_mask_to_blocks(selected_mask, k_selected, local_window=1):
     out = torch.empty((1, L, G, qb, width), device=mask.device, dtype=torch.int32)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(mask.device):
+    with spruce_hip.on_device(mask.device):
         rc = spruce_hip.lib().spruce_pack_selected_mask(
             mask.data_ptr(), L * G * qb, qb, kb, int(k_selected), int(local_window),
             out.data_ptr(), width, spruce_hip.stream_of(mask))
@@ -88,7 +88,7 @@ def selected_ids_to_blocks(selected_ids, k_selected, local_window=1, key_blocks=
     out = torch.empty((1, L, G, qb, width), device=ids.device, dtype=torch.int32)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(ids.device):
+    with spruce_hip.on_device(ids.device):
         rc = spruce_hip.lib().spruce_pack_selected_ids(
             ids.data_ptr(), ids.element_size(), L * G * qb, qb, C, kb, int(k_selected),
             int(local_window), int(sink_blocks), out.data_ptr(), width, spruce_hip.stream_of(ids))

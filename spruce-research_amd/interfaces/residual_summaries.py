@@ -172,7 +172,7 @@ def build_residual_summary_nodes(selected_blocks: torch.Tensor, *,
     sel = selected_blocks.to(dev)
     counts = torch.empty(rows, dtype=torch.int32, device=dev)
     lib = spruce_hip.lib()
-    with torch.cuda.device(dev):
+    with spruce_hip.on_device(dev):
         stream = spruce_hip.stream_of(sel)
         args = (spruce_hip.ptr(sel), spruce_hip.strides5(sel), batch, layers, groups, query_blocks, width)
         spruce_hip.check(lib.spruce_residual_frontier(*args, spruce_hip.ptr(counts), None, 0, stream),

@@ -50,7 +50,7 @@ def block_sparse_prefill(q, k, v, block_mask, scale, block_size=64,
         raise ValueError("block_mask must be on the same device as q")
     mask_u8 = block_mask.view(torch.uint8) if block_mask.dtype == torch.bool else block_mask
     out = torch.empty((B, Hq, T, D), device=q.device, dtype=q.dtype)
-    with torch.cuda.device(q.device):
+    with spruce_hip.on_device(q.device):
         rc = spruce_hip.lib().spruce_sparse_prefill_mask(
             spruce_hip.ptr(q), spruce_hip.strides(q),
             spruce_hip.ptr(k), spruce_hip.strides(k),

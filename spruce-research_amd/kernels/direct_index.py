@@ -49,8 +49,9 @@ def _output(q):
 
 
 def _record(kernel_variant, Hq, Hkv, D):
-    _LAST_CONFIG[kernel_variant] = spruce_hip.launch_config(
-        kernel_variant, Hq, Hkv, D)["best_config"]
+    # The configuration is worked out when kernel_runtime_metadata asks for it
+    # (11 us of host time, half of a short prompt's call).
+    _LAST_CONFIG[kernel_variant] = (Hq, Hkv, D)
 
 
 def _key_valid(key_valid, B, T, device):
@@ -113,7 +114,7 @@ def direct_index_sparse_prefill(q, k, v, indices, scale, block_size=64,
             raise ValueError("pass either key_valid or attn_mask, not both")
         mask, code = _attn_mask(attn_mask, B, Hq, T, q.device)
         mview = mask.view(torch.uint8) if mask.dtype == torch.bool else mask
-        with torch.cuda.device(q.device):
+        with spruce_hip.on_device(q.device):
             rc = spruce_hip.lib().spruce_sparse_prefill_index_amask(
                 spruce_hip.ptr(q), spruce_hip.strides(q),
                 spruce_hip.ptr(k), spruce_hip.strides(k),
@@ -129,7 +130,7 @@ def direct_index_sparse_prefill(q, k, v, indices, scale, block_size=64,
     if key_valid is not None:
         kv8 = _key_valid(key_valid, B, T, q.device)
         zero4 = spruce_hip.strides(torch.empty(0, 0, 0, 0))
-        with torch.cuda.device(q.device):
+        with spruce_hip.on_device(q.device):
             rc = spruce_hip.lib().spruce_sparse_prefill_index_masked(
                 spruce_hip.ptr(q), spruce_hip.strides(q),
                 spruce_hip.ptr(k), spruce_hip.strides(k),
@@ -143,7 +144,7 @@ def direct_index_sparse_prefill(q, k, v, indices, scale, block_size=64,
         spruce_hip.check(rc, "spruce_sparse_prefill_index_masked")
         _record(kernel_variant, Hq, Hkv, D)
         return out
-    with torch.cuda.device(q.device):
+    with spruce_hip.on_device(q.device):
         rc = spruce_hip.lib().spruce_sparse_prefill_index(
             spruce_hip.ptr(q), spruce_hip.strides(q),
             spruce_hip.ptr(k), spruce_hip.strides(k),
@@ -195,7 +196,7 @@ def direct_index_sparse_summaries(q, k, v, indices, nodes, table, scale, block_s
     out, out_strides = _output(q)
     if key_valid is not None:
         kv8 = _key_valid(key_valid, B, T, q.device)
-        with torch.cuda.device(q.device):
+        with spruce_hip.on_device(q.device):
             rc = spruce_hip.lib().spruce_sparse_prefill_index_masked(
                 spruce_hip.ptr(q), spruce_hip.strides(q),
                 spruce_hip.ptr(k), spruce_hip.strides(k),
@@ -211,7 +212,7 @@ def direct_index_sparse_summaries(q, k, v, indices, nodes, table, scale, block_s
         spruce_hip.check(rc, "spruce_sparse_prefill_index_masked")
         _record(kernel_variant, Hq, Hkv, D)
         return out
-    with torch.cuda.device(q.device):
+    with spruce_hip.on_device(q.device):
         rc = spruce_hip.lib().spruce_sparse_prefill_index_summaries(
             spruce_hip.ptr(q), spruce_hip.strides(q),
             spruce_hip.ptr(k), spruce_hip.strides(k),
@@ -255,7 +256,7 @@ def direct_index_sparse_csr(q, k, v, indptr, indices, scale, block_size=64,
         if t.device != q.device:
             raise ValueError("index tensors must be on the same device as q")
     out, out_strides = _output(q)
-    with torch.cuda.device(q.device):
+    with spruce_hip.on_device(q.device):
         rc = spruce_hip.lib().spruce_sparse_prefill_csr(
             spruce_hip.ptr(q), spruce_hip.strides(q),
             spruce_hip.ptr(k), spruce_hip.strides(k),
@@ -298,4 +299,6 @@ def kernel_runtime_metadata(kernel_variant):
         raise ValueError(
             f"kernel_variant must be one of {KERNEL_VARIANTS}, "
             f"got {kernel_variant!r}")
-    return {"variant": kernel_variant, "best_config": _LAST_CONFIG.get(kernel_variant)}
+    shape = _LAST_CONFIG.get(kernel_variant)
+    config = spruce_hip.launch_config(kernel_variant, *shape)["best_config"] if shape else None
+    return {"variant": kernel_variant, "best_config": config}

@@ -96,7 +96,7 @@ class FlatGate(nn.Module):
         out = torch.empty((L, G, qb, C), device=qp.device, dtype=torch.float32)
         if C == 0:
             return out
-        with torch.cuda.device(qp.device):
+        with spruce_hip.on_device(qp.device):
             rc = spruce_hip.lib().spruce_gate_candidate_scores(
                 spruce_hip.ptr(qp), spruce_hip.ptr(kp), spruce_hip.ptr(ids), L * G, qb, N, C,
                 qp.shape[3], Pk, p, float(math.sqrt(self.proj_dim)), spruce_hip.ptr(out),

@@ -55,7 +55,7 @@ def pool_blocks(query=None, key=None):
     nb = (T + BLOCK - 1) // BLOCK
     q_mean = torch.empty((B, Hkv, nb, D), device=key.device, dtype=torch.float32) if query is not None else None
     k_sum = torch.empty((B, Hkv, nb, 2, D), device=key.device, dtype=torch.float32)
-    with torch.cuda.device(key.device):
+    with spruce_hip.on_device(key.device):
         rc = spruce_hip.lib().spruce_selector_pool(
             spruce_hip.ptr(query), spruce_hip.strides(query) if query is not None else None,
             spruce_hip.ptr(key), spruce_hip.strides(key),
@@ -107,7 +107,7 @@ def pool_project(query, key, Wq, Wk):
     Wk = Wk.to(query.device).contiguous()
     qp = torch.empty((B, Hkv, nb, P), device=query.device, dtype=torch.float32)
     kp = torch.empty((B, Hkv, nb, 2, P), device=query.device, dtype=torch.float32)
-    with torch.cuda.device(query.device):
+    with spruce_hip.on_device(query.device):
         rc = spruce_hip.lib().spruce_selector_pool_project(
             spruce_hip.ptr(query), spruce_hip.strides(query), spruce_hip.ptr(key), spruce_hip.strides(key),
             B, Hq, Hkv, T, D, spruce_hip.dtype_code(query), spruce_hip.ptr(Wq), spruce_hip.ptr(Wk), P,
@@ -128,7 +128,7 @@ def project(x, W):
     N, D = x2.shape
     P = W.shape[1]
     out = torch.empty((N, P), device=x.device, dtype=torch.float32)
-    with torch.cuda.device(x.device):
+    with spruce_hip.on_device(x.device):
         rc = spruce_hip.lib().spruce_gate_project(
             spruce_hip.ptr(x2), spruce_hip.ptr(W), N, D, P, spruce_hip.ptr(out), spruce_hip.stream_of(x))
     spruce_hip.check(rc, "spruce_gate_project")
@@ -177,7 +177,7 @@ def project_layers(levels, W, interleaved=False):
     out = torch.empty(shape, device=bufs[0].device, dtype=torch.float32)
     ptrs = (ctypes.c_void_p * len(bufs))(*[t.data_ptr() for t in bufs])
     counts = (ctypes.c_int64 * len(bufs))(*nodes)
-    with torch.cuda.device(bufs[0].device):
+    with spruce_hip.on_device(bufs[0].device):
         rc = spruce_hip.lib().spruce_gate_project_layers(
             ptrs, counts, len(bufs), L, S, P, D, spruce_hip.dtype_code(bufs[0]), spruce_hip.ptr(W), p,
             spruce_hip.ptr(out), 1 if interleaved else 0, spruce_hip.stream_of(bufs[0]))
@@ -203,7 +203,7 @@ def project_pair(xa, Wa, xb, Wb):
     D, P = Wa.shape
     oa = torch.empty((xa2.shape[0], P), device=xa.device, dtype=torch.float32)
     ob = torch.empty((xb2.shape[0], P), device=xa.device, dtype=torch.float32)
-    with torch.cuda.device(xa.device):
+    with spruce_hip.on_device(xa.device):
         rc = spruce_hip.lib().spruce_gate_project2(
             spruce_hip.ptr(xa2), spruce_hip.ptr(Wa), xa2.shape[0], spruce_hip.ptr(xb2), spruce_hip.ptr(Wb),
             xb2.shape[0], D, P, spruce_hip.ptr(oa), spruce_hip.ptr(ob), spruce_hip.stream_of(xa))
@@ -228,7 +228,7 @@ def gate_scores(qp, kp, causal=True, div=None):
     Kb, Pk = kp.shape[1], kp.shape[2]
     d = math.sqrt(P) if div is None else float(div)
     out = torch.empty((S, Qb, Kb), device=qp.device, dtype=torch.float32)
-    with torch.cuda.device(qp.device):
+    with spruce_hip.on_device(qp.device):
         rc = spruce_hip.lib().spruce_gate_scores(
             spruce_hip.ptr(qp), spruce_hip.ptr(kp), S, Qb, Kb, Pq, Pk, P, d,
             2 if causal == "lower" else int(bool(causal)),
@@ -249,7 +249,7 @@ def causal_topk_blocks(scores, k):
     s = scores.reshape(-1, Qb, Kb).contiguous()
     R = s.shape[0]
     out = torch.empty((R, Qb, k), device=scores.device, dtype=torch.int32)
-    with torch.cuda.device(scores.device):
+    with spruce_hip.on_device(scores.device):
         rc = spruce_hip.lib().spruce_causal_topk(
             spruce_hip.ptr(s), R, Qb, Kb, k, spruce_hip.ptr(out), spruce_hip.stream_of(scores))
     spruce_hip.check(rc, "spruce_causal_topk")
@@ -299,7 +299,7 @@ def select_blocks_fused(query, key, Wq, Wk, top_k=32):
     nbytes = lib.spruce_select_flat_workspace_bytes(B, Hkv, T, P)
     ws = torch.empty(nbytes // 4, device=query.device, dtype=torch.float32)
     out = torch.empty((B, Hkv, nb, top_k), device=query.device, dtype=torch.int32)
-    with torch.cuda.device(query.device):
+    with spruce_hip.on_device(query.device):
         rc = lib.spruce_select_flat(
             spruce_hip.ptr(query), spruce_hip.strides(query), spruce_hip.ptr(key), spruce_hip.strides(key),
             B, Hq, Hkv, T, D, spruce_hip.dtype_code(query), spruce_hip.ptr(Wq), spruce_hip.ptr(Wk), P,

@@ -72,7 +72,7 @@ def traverse_projected(projected_q, projected_k_all, num_leaves, beam, radix, di
     kp = projected_k_all.float().contiguous()
     C = output_width(num_leaves, radix, beam)
     out = torch.empty((L, G, qb, C), device=qp.device, dtype=torch.int32)
-    with torch.cuda.device(qp.device):
+    with spruce_hip.on_device(qp.device):
         rc = spruce_hip.lib().spruce_tree_traverse(
             spruce_hip.ptr(qp), spruce_hip.ptr(kp), L * G, qb, num_leaves, Pq, Pk, p, radix, beam,
             float(div), spruce_hip.ptr(out), C, 1 if interleaved else 0, spruce_hip.stream_of(qp))

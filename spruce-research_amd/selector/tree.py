@@ -118,7 +118,7 @@ def merge_level(features, radix=2):
     L, G, n, P, d = features.shape
     x = features.contiguous()
     out = torch.empty((L, G, (n + radix - 1) // radix, P, d), device=x.device, dtype=x.dtype)
-    with torch.cuda.device(x.device):
+    with spruce_hip.on_device(x.device):
         rc = spruce_hip.lib().spruce_tree_merge_level(
             spruce_hip.ptr(x), L * G, n, P, d, radix, spruce_hip.dtype_code(x), spruce_hip.ptr(out),
             spruce_hip.stream_of(x))
@@ -145,7 +145,7 @@ def merge_levels(features, radix=2):
     if not outs:
         return outs
     ptrs = (ctypes.c_void_p * len(outs))(*[o.data_ptr() for o in outs])
-    with torch.cuda.device(x.device):
+    with spruce_hip.on_device(x.device):
         rc = spruce_hip.lib().spruce_tree_merge_levels(
             spruce_hip.ptr(x), L * G, x.shape[2], P, d, radix, spruce_hip.dtype_code(x), ptrs, len(outs),
             spruce_hip.stream_of(x))

@@ -187,7 +187,7 @@ def _key_validity_and_padding(attention_mask: torch.Tensor, batch: int, seq_len:
         return valid, valid is not None and not bool(valid.all())
     valid = torch.empty((batch, seq_len), device=m.device, dtype=torch.bool)
     flags = torch.zeros(2, device=m.device, dtype=torch.int32)
-    with torch.cuda.device(m.device):
+    with spruce_hip.on_device(m.device):
         rc = spruce_hip.lib().spruce_mask_key_validity(
             spruce_hip.ptr(m), spruce_hip.strides(m), m.shape[1], _MASK_CODES[m.dtype], batch, seq_len,
             spruce_hip.ptr(valid), spruce_hip.ptr(flags), spruce_hip.stream_of(m))

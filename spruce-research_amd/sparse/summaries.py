@@ -99,7 +99,7 @@ def build_kv_summary_table(key: torch.Tensor, value: torch.Tensor, layout: Resid
     nbytes = spruce_hip.lib().spruce_kv_summary_workspace_bytes(batch, kv_heads, seq_len, head_dim)
     ws = torch.empty(max(nbytes, 1), device=dev, dtype=torch.uint8)
     s_flat, e_flat = starts.contiguous().view(-1), ends.contiguous().view(-1)
-    with torch.cuda.device(dev):
+    with spruce_hip.on_device(dev):
         rc = spruce_hip.lib().spruce_kv_summary(
             spruce_hip.ptr(key), spruce_hip.strides(key), spruce_hip.ptr(value), spruce_hip.strides(value),
             batch, kv_heads, seq_len, head_dim, spruce_hip.dtype_code(key), spruce_hip.ptr(valid),

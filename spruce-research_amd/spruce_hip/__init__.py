@@ -10,6 +10,7 @@ torch is imported before the library is opened so that the library binds to
 the HIP runtime torch already loaded (both carry the SONAME
 ``libamdhip64.so.7``), keeping one runtime and one set of streams per process.
 """
+import contextlib
 import ctypes
 import json
 import os
@@ -165,12 +166,15 @@ def check(rc, what):
     raise RuntimeError(f"{what} failed with hipError {rc}: {message}")
 
 
+_I64X4 = _i64 * 4
+
+
 def strides(t, order=None):
     """int64[4] element strides of a 4-D tensor (optionally permuted)."""
-    s = t.stride() if order is None else tuple(t.stride(i) for i in order)
+    s = t.stride()
     if len(s) != 4:
         raise ValueError(f"expected a 4-D tensor, got {t.dim()}-D")
-    return (_i64 * 4)(*s)
+    return _I64X4(*s) if order is None else _I64X4(*[s[i] for i in order])
 
 
 def strides5(t):
@@ -181,11 +185,21 @@ def strides5(t):
 
 
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def stream_of(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return torch.cuda.current_stream(t.device).cuda_stream
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def on_device(device):
+    """``torch.cuda.device(device)``, and nothing where it is current already."""
+    if device.index == torch.cuda.current_device():
+        return _SAME_DEVICE
+    return torch.cuda.device(device)
 
 
 def dtype_code(t):

@@ -72,7 +72,7 @@ def block_mass(query, key, scaling, block_size=_BLOCK, schedule="auto"):
         spruce_hip.check(code if code < 0 else 0, "spruce_teacher_schedule")
     nbytes = lib.spruce_teacher_schedule_workspace_bytes(b, H, q_len, code)
     ws = torch.empty((nbytes + 3) // 4, device=query.device, dtype=torch.float32)
-    with torch.cuda.device(query.device):
+    with spruce_hip.on_device(query.device):
         rc = lib.spruce_teacher_block_mass_schedule(
             spruce_hip.ptr(query), spruce_hip.strides(query), spruce_hip.ptr(key), spruce_hip.strides(key),
             b, H, Hkv, q_len, d, float(scaling), spruce_hip.dtype_code(query),
@@ -102,7 +102,7 @@ def _launch_proto(x, G, block, P):
     out = torch.empty((b, G, nb, P, d), device=x.device, dtype=x.dtype)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(x.device):
+    with spruce_hip.on_device(x.device):
         rc = spruce_hip.lib().spruce_proto_pool(
             spruce_hip.ptr(x), spruce_hip.strides(x), b, H, L, d, G, block, P,
             spruce_hip.dtype_code(x), spruce_hip.ptr(out), spruce_hip.stream_of(x))
@@ -149,7 +149,7 @@ def proto_pool_qk(query, key, block=_BLOCK, P=_PROTO):
     nb = (L + block - 1) // block
     out_q = torch.empty((b, G, nb, P, d), device=query.device, dtype=query.dtype)
     out_k = torch.empty((b, G, nb, P, d), device=query.device, dtype=query.dtype)
-    with torch.cuda.device(query.device):
+    with spruce_hip.on_device(query.device):
         rc = spruce_hip.lib().spruce_proto_pool_qk(
             spruce_hip.ptr(query), spruce_hip.strides(query), spruce_hip.ptr(key), spruce_hip.strides(key),
             b, H, G, L, d, block, P, spruce_hip.dtype_code(query), spruce_hip.ptr(out_q), spruce_hip.ptr(out_k),
@@ -170,7 +170,7 @@ def _group_avg_tokens(x, G):
     out = torch.empty((b, G, L, d), device=x.device, dtype=x.dtype)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(x.device):
+    with spruce_hip.on_device(x.device):
         rc = spruce_hip.lib().spruce_group_avg_tokens(
             spruce_hip.ptr(x), spruce_hip.strides(x), b, H, L, d, G,
             spruce_hip.dtype_code(x), spruce_hip.ptr(out), spruce_hip.stream_of(x))
@@ -211,7 +211,7 @@ def causal_prefill_features(query, key, value, scaling, P=_PROTO, capture=True):
         q_grouped = torch.empty((B, G, L, d), device=query.device, dtype=query.dtype)
         k_protos = torch.empty((B, G, nb, P, d), device=query.device, dtype=query.dtype)
     out, out_strides = _output(query)
-    with torch.cuda.device(query.device):
+    with spruce_hip.on_device(query.device):
         rc = spruce_hip.lib().spruce_causal_prefill(
             spruce_hip.ptr(query), spruce_hip.strides(query), spruce_hip.ptr(key), spruce_hip.strides(key),
             spruce_hip.ptr(value), spruce_hip.strides(value), B, H, G, L, d, float(scaling),

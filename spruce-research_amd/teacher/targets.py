@@ -28,7 +28,7 @@ def teacher_targets(mass, num_kv_heads, k=8, eps=1e-9):
     target = torch.empty((B, G, Qb, Kb), device=mass.device, dtype=torch.float32)
     row_mass = torch.empty((B, G, Qb), device=mass.device, dtype=torch.float32)
     topk = torch.empty((B, G, Qb, k), device=mass.device, dtype=torch.int32)
-    with torch.cuda.device(mass.device):
+    with spruce_hip.on_device(mass.device):
         rc = spruce_hip.lib().spruce_teacher_targets(
             spruce_hip.ptr(mass), B, H, G, Qb, Kb, k, float(eps), spruce_hip.ptr(target),
             spruce_hip.ptr(row_mass), spruce_hip.ptr(topk), spruce_hip.stream_of(mass))
@@ -53,7 +53,7 @@ def teacher_group_mass(mass, num_kv_heads):
     mass = mass.contiguous()
     out = torch.empty((B, G, Qb, Kb), device=mass.device, dtype=torch.float32)
     row_mass = torch.empty((B, G, Qb), device=mass.device, dtype=torch.float32)
-    with torch.cuda.device(mass.device):
+    with spruce_hip.on_device(mass.device):
         rc = spruce_hip.lib().spruce_teacher_group_mass(
             spruce_hip.ptr(mass), B, H, G, Qb, Kb, spruce_hip.ptr(out), spruce_hip.ptr(row_mass),
             spruce_hip.stream_of(mass))
