@@ -101,6 +101,7 @@ struct AttnParams {
   const float* slog;
   float sbias;  // log counts -> raw score units: log2(e) / cs
   int tpp;  // tiles per part: waves 0..tpp-1 of a workgroup own a tile
+  int help;  // small grid: as many helper waves as tile waves (4- and 2-tile parts)
   // feature capture (dense causal form): group-averaged queries
   // [B, Hkv, T, D] and key prototypes [B, Hkv, Qb, P, D], model dtype,
   // contiguous; each part covers tpp / G whole 32-row halves of the block.
@@ -537,16 +538,30 @@ __device__ __forceinline__ void amask_unpack4(int dt, const uint4& x, float (&v)
   }
 }
 
+// Workgroup barrier that orders LDS only: the global loads a wave has in
+// flight stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// HELP: the second half of the workgroup's waves own no tile and stage every
+// K/V block through their registers, a block ahead of the one the tile waves
+// compute.  In a small grid a tile wave has its SIMD to itself, so what bounds
+// it is its own chain per block; the wait for the staged loads, the rounding
+// of float32 blocks and the LDS stores leave that chain.
 template <int D, int WAVES, typename TIn, bool F16, int MODE, bool SUMM = false, bool CAP = false, bool PROD = false,
-          bool KVAL = false, bool AMASK = false>
-__global__ __launch_bounds__(WAVES * 64) void sparse_prefill_kernel(const AttnParams p) {
+          bool KVAL = false, bool AMASK = false, bool HELP = false>
+__global__ __launch_bounds__(WAVES * 64, HELP && !AMASK ? 2 : 1) void sparse_prefill_kernel(const AttnParams p) {
   static_assert(!CAP || (MODE == kModeCausal && !SUMM && TIn::bytes == 2),
                 "feature capture runs on the dense causal form in the model dtype");
   static_assert(!KVAL || MODE == kModePadded, "key padding is supported for padded block lists");
   static_assert(!AMASK || (MODE == kModePadded && !SUMM && !KVAL && !CAP),
                 "the general attention mask is supported for padded block lists without summaries");
   static_assert(!PROD || TIn::bytes == 2, "the producer form stages 16-bit K/V");
-  constexpr int NTHR = WAVES * 64;
+  static_assert(!HELP || (!PROD && !SUMM && !CAP), "helper waves stage key blocks only");
+  constexpr int NTHR = HELP ? WAVES * 32 : WAVES * 64;  // threads that stage a block
   constexpr int KSTR = D + 8;        // K tile row stride, 16-bit elements (16 B pad)
   // V tile row stride: rows start 16 banks apart, so the 8 rows x 64 bytes
   // a transposing read touches fall in distinct banks per half-wave.
@@ -656,9 +671,10 @@ __global__ __launch_bounds__(WAVES * 64) void sparse_prefill_kernel(const AttnPa
   const char* vbase = static_cast<const char*>(p.v) + ((int64_t)b * p.vs[0] + (int64_t)g * p.vs[1]) * EB;
   const int krs = (int)(p.ks[2] * EB), vrs = (int)(p.vs[2] * EB);
   int koff[KCH], klds[KCH];
+  const int stid = HELP ? tid & (NTHR - 1) : tid;
 #pragma unroll
   for (int i = 0; i < KCH; ++i) {
-    const int c = tid + i * NTHR;
+    const int c = stid + i * NTHR;
     const int key = c / KROWCH, dc = c % KROWCH;
     koff[i] = c < KCHUNKS ? key * krs + dc * 8 * EB : kOutOfRange;
     klds[i] = key * KSTR + dc * 8;
@@ -666,7 +682,7 @@ __global__ __launch_bounds__(WAVES * 64) void sparse_prefill_kernel(const AttnPa
   int voff[KCH], vlds[KCH];
 #pragma unroll
   for (int i = 0; i < KCH; ++i) {
-    const int c = tid + i * NTHR;
+    const int c = stid + i * NTHR;
     const int key = c / KROWCH, dc = c % KROWCH;
     voff[i] = c < KCHUNKS ? key * vrs + dc * 8 * EB : kOutOfRange;
     vlds[i] = key * VSTR + dc * 8;
@@ -692,7 +708,7 @@ __global__ __launch_bounds__(WAVES * 64) void sparse_prefill_kernel(const AttnPa
     uint16_t* Vs = Ks + KTILE;
 #pragma unroll
     for (int i = 0; i < KCH; ++i) {
-      if ((KCHUNKS % NTHR) == 0 || tid + i * NTHR < KCHUNKS) {
+      if ((KCHUNKS % NTHR) == 0 || stid + i * NTHR < KCHUNKS) {
         *reinterpret_cast<uint4*>(Ks + klds[i]) = raw_to_mfma<TIn, F16>(kst[i]);
         *reinterpret_cast<uint4*>(Vs + vlds[i]) = raw_to_mfma<TIn, F16>(vst[i]);
       }
@@ -799,7 +815,7 @@ __global__ __launch_bounds__(WAVES * 64) void sparse_prefill_kernel(const AttnPa
   uint4 amr[AMASK ? 8 : 1];
   bool am_rows = false;  // wave-uniform: amr holds row pieces
   constexpr int kAmRowWords = 68;  // LDS row of the staging region: 256 + 16 bytes
-  __shared__ __attribute__((aligned(16))) uint32_t amlds[AMASK ? WAVES * 32 * kAmRowWords : 1];
+  __shared__ __attribute__((aligned(16))) uint32_t amlds[AMASK ? (HELP ? WAVES / 2 : WAVES) * 32 * kAmRowWords : 1];
   auto fetch_amask = [&](int blk) {
     if constexpr (AMASK) {
 #pragma unroll
@@ -1172,6 +1188,47 @@ __global__ __launch_bounds__(WAVES * 64) void sparse_prefill_kernel(const AttnPa
         vcur = vnext;
       }
     }
+  } else if constexpr (HELP) {
+    // One barrier before the first block and one between consecutive blocks
+    // on both sides.  In the period in which the tile waves compute block i
+    // the helpers store block i + 1, loaded a period ago, and issue block
+    // i + 2's loads.
+    if (wave >= WAVES / 2) {
+      if (any_block) {
+        load_block(cur_id);
+        int nid = 0;
+        bool nen = false;
+        store_block(0);
+        bool more = it.next(nid, nen);
+        if (more) load_block(nid);
+        lds_barrier();
+        while (more) {
+          store_block(buf ^ 1);
+          more = it.next(nid, nen);
+          if (more) load_block(nid);
+          lds_barrier();
+          buf ^= 1;
+        }
+      }
+    } else if (any_block) {
+      uint32_t vcur = vbyte(cur_id);
+      fetch_amask(cur_id);
+      if (!q_ready) convert_q();
+      lds_barrier();
+      while (true) {
+        int nid = 0;
+        bool nen = false;
+        const bool more = it.next(nid, nen);
+        const uint32_t vnext = more ? vbyte(nid) : 0u;
+        if (active && cur_en) compute(buf, cur_id == qb, nullptr, vbits(vcur), more ? nid : -1);
+        if (!more) break;
+        lds_barrier();
+        buf ^= 1;
+        cur_id = nid;
+        cur_en = nen;
+        vcur = vnext;
+      }
+    }
   } else if (any_block) {
     uint32_t vcur = vbyte(cur_id);
     load_block(cur_id);
@@ -1361,7 +1418,15 @@ inline LaunchShape choose_shape(int variant, int G) {
 // has one, since a second fetch of a row's K/V blocks costs less than an
 // idle CU.  Every shape computes the same attention.
 constexpr int64_t kComputeUnits = 256;  // MI355X
-inline void split_small_grid(AttnParams& p, LaunchShape& s, int variant) {
+//
+// Helper waves (the HELP form) double a 4- or 2-tile workgroup; they are taken
+// while the grid still leaves every SIMD at most two waves (one workgroup of
+// eight waves or two of four on a CU; `one_per_cu`: a form whose LDS lets only
+// one workgroup on a CU).  Measured (index form, before ->
+// after): 8/2 heads, T = 4096, 27 blocks a row, float32 58.0 -> 41.1, bf16 47.4
+// -> 34.5 us; 12/2, T = 333, 6 blocks 13.6 -> 10.5; 28/4, T = 1000, 10 blocks
+// 21.8 -> 19.6.
+inline void split_small_grid(AttnParams& p, LaunchShape& s, int variant, bool one_per_cu = false) {
   if (variant == SPRUCE_VARIANT_SINGLE_HEAD_QTILE) return;
   const int64_t rows = (int64_t)p.B * p.Hkv * p.Qb;
   const int tiles = 2 * p.G;
@@ -1373,21 +1438,28 @@ inline void split_small_grid(AttnParams& p, LaunchShape& s, int variant) {
   }
   p.parts = s.parts;
   p.tpp = s.tpp;
+  const int64_t per_cu = one_per_cu || s.waves == 4 ? 1 : 2;
+  p.help = s.waves < 8 && s.tpp == s.waves && rows * s.parts <= kComputeUnits * per_cu;
 }
 
 template <int D, int WAVES, typename TIn, bool F16, int MODE, bool SUMM, bool CAP = false, bool PROD = false,
-          bool KVAL = false, bool AMASK = false>
+          bool KVAL = false, bool AMASK = false, bool HELP = false>
 int launch_attention_t(const AttnParams& p, hipStream_t stream) {
   // Rows are padded to a multiple of the 8 XCDs; the extra workgroups exit.
   const int64_t rows8 = ((int64_t)p.B * p.Hkv * p.Qb + 7) / 8 * 8;
   const int64_t grid = rows8 * p.parts;
-  hipLaunchKernelGGL((sparse_prefill_kernel<D, WAVES, TIn, F16, MODE, SUMM, CAP, PROD, KVAL, AMASK>),
+  hipLaunchKernelGGL((sparse_prefill_kernel<D, WAVES, TIn, F16, MODE, SUMM, CAP, PROD, KVAL, AMASK, HELP>),
                      dim3((unsigned)grid), dim3(WAVES * 64), 0, stream, p);
   return check_launch("sparse_prefill_kernel");
 }
 
 template <int MODE, bool SUMM, int D, typename TIn, bool F16, bool KVAL, bool AMASK = false>
 int launch_attention_w(const AttnParams& p, int waves, hipStream_t stream) {
+  if constexpr (!SUMM && MODE != kModeCausal)
+    if (p.help) {
+      if (waves == 2) return launch_attention_t<D, 4, TIn, F16, MODE, false, false, false, KVAL, AMASK, true>(p, stream);
+      if (waves == 4) return launch_attention_t<D, 8, TIn, F16, MODE, false, false, false, KVAL, AMASK, true>(p, stream);
+    }
   switch (waves) {
     case 2: return launch_attention_t<D, 2, TIn, F16, MODE, SUMM, false, false, KVAL, AMASK>(p, stream);
     case 4: return launch_attention_t<D, 4, TIn, F16, MODE, SUMM, false, false, KVAL, AMASK>(p, stream);

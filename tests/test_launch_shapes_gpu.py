@@ -137,3 +137,64 @@ def test_split_and_unsplit_launches_agree(entry, Hq, Hkv, B, dtype):
         alone, first = _alone_and_first(call, (q, k, v, selected, residual))
     assert torch.isfinite(alone.float()).all()
     assert torch.equal(alone, first), (entry, (alone.float() - first.float()).abs().max().item())
+
+
+@pytest.mark.parametrize("dtype,head_dim", [(torch.bfloat16, 128), (torch.float16, 64), (torch.float32, 128)])
+@pytest.mark.parametrize("Hq,Hkv,tokens,variant", [
+    (8, 2, 4096, "single_head"),        # 128 rows: 4-tile parts with helper waves fill 256 CUs exactly
+    (8, 2, 4100, "single_head"),        # one row more: no helper waves
+    (12, 2, 333, "single_head"),        # 2-tile parts with helper waves, ragged
+    (28, 4, 1170, "single_head"),       # 2-tile parts, 532 workgroups: no helper waves
+    (2, 1, 8, "single_head"),           # one row of one block
+    (8, 2, 600, "single_head_qtile"),   # keeps its own shape
+])
+def test_helper_wave_launches_agree_with_the_eight_wave_forms(Hq, Hkv, tokens, variant, dtype, head_dim):
+    # Small grids take helper waves (or just miss them); batch element 0 must
+    # equal the one of a batch that fills the GPU, for every list form, with
+    # empty rows, rows of one block and rows of several.
+    print(f"helper waves: Hq={Hq} Hkv={Hkv} T={tokens} D={head_dim} {dtype} {variant}", flush=True)
+    qb = (tokens + 63) // 64
+    B = max(2, -(-512 // (Hkv * qb)))
+    B = min(B, 12)
+    gen = torch.Generator().manual_seed(tokens + Hq)
+    q, k, v = [torch.randn(B, tokens, H, head_dim, generator=gen).to(dtype).to(DEV).transpose(1, 2)
+               for H in (Hq, Hkv, Hkv)]
+    scale = head_dim ** -0.5
+    keep = torch.rand(B, Hkv, qb, qb, generator=gen) < min(1.0, 5.0 / qb)
+    keep |= torch.eye(qb, dtype=torch.bool)
+    keep &= torch.ones(qb, qb).tril().bool()
+    if qb > 2:
+        keep[:, :, qb // 2] &= torch.arange(qb) == 0
+        keep[:, :, qb // 3] = False
+    width = int(keep.sum(-1).max())
+    ids = torch.where(keep, torch.arange(qb), qb).sort(-1).values[..., :width]
+    idx = torch.where(ids == qb, -1, ids).to(torch.int32).contiguous().to(DEV)
+    mask = keep.repeat_interleave(Hq // Hkv, 1).to(DEV)
+    counts = keep.sum(-1).reshape(-1)
+    ptr = torch.cat([torch.zeros(1, dtype=torch.long), counts.cumsum(0)]).int()
+    ind = keep.nonzero()[:, 3].int()
+    n1 = Hkv * qb
+    valid = (torch.arange(tokens)[None] >= torch.randint(0, tokens // 2 + 1, (B, 1), generator=gen)).to(DEV)
+    bias = torch.randn(B, 1, tokens, tokens, generator=gen).to(torch.bfloat16).to(DEV) if tokens <= 1200 else None
+    kw = dict(kernel_variant=variant)
+    pairs = {
+        "index": (direct_index_sparse_prefill(q[:1], k[:1], v[:1], idx[:1], scale, **kw),
+                  direct_index_sparse_prefill(q, k, v, idx, scale, **kw)),
+        "mask": (block_sparse_prefill(q[:1], k[:1], v[:1], mask[:1], scale, **kw),
+                 block_sparse_prefill(q, k, v, mask, scale, **kw)),
+        "csr": (direct_index_sparse_csr(q[:1], k[:1], v[:1], ptr[: n1 + 1].to(DEV), ind[: int(ptr[n1])].to(DEV),
+                                        scale, **kw),
+                direct_index_sparse_csr(q, k, v, ptr.to(DEV), ind.to(DEV), scale, **kw)),
+        "key_valid": (direct_index_sparse_prefill(q[:1], k[:1], v[:1], idx[:1], scale, key_valid=valid[:1], **kw),
+                      direct_index_sparse_prefill(q, k, v, idx, scale, key_valid=valid, **kw)),
+    }
+    if bias is not None:
+        pairs["attn_mask"] = (
+            direct_index_sparse_prefill(q[:1], k[:1], v[:1], idx[:1], scale, attn_mask=bias[:1], **kw),
+            direct_index_sparse_prefill(q, k, v, idx, scale, attn_mask=bias, **kw))
+    torch.cuda.synchronize()
+    for name, (alone, together) in pairs.items():
+        assert torch.isfinite(alone.float()).all(), name
+        assert torch.equal(alone, together[:1]), name
+    assert torch.equal(pairs["index"][0], pairs["mask"][0].transpose(1, 2))
+    assert torch.equal(pairs["index"][0], pairs["csr"][0])
