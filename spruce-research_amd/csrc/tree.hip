@@ -183,6 +183,119 @@ __device__ __forceinline__ void merge_parent(const MergeParams& p, int64_t s, in
   }
 }
 
+// Four parents per wavefront, 16 lanes each, for 16-bit features of D = 64 or
+// 128 dims and at most 16 candidates (radix * P), 16-byte aligned.  Lane i of
+// a group holds candidate i's whole row in registers, so its distance chain
+// (dims in order) reads nothing but the mean; the mean is formed 8 dims a lane
+// from the children's prototype 0 and passed through LDS; ranks count over the
+// group by DPP rotations; and the P - 1 chosen lanes store the rows they hold.
+// The values are merge_parent's.
+//
+// Bound: one parent's chain (a load round trip, D dependent adds, a store):
+// levels are formed one after the other, and the lower ones fill the CUs.  At
+// 2048 leaves x 4 slabs of 8 x 128 bf16 the eleven levels take 75 us (one parent a
+// wavefront, features and distances through LDS: 117 us).
+template <bool F16>
+__device__ __forceinline__ float round16(float x) {
+  if constexpr (F16) return (float)(_Float16)x;
+  else return (float)(__bf16)x;
+}
+
+// f(1), f(2), ... as integral constants.
+template <typename F, int... I>
+__device__ __forceinline__ void for_each_index(F& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I + 1>{}), ...);
+}
+
+template <bool F16, int D>
+__device__ __forceinline__ void merge_four(const MergeParams& p, int64_t s, int j, bool live, int lane, float* sh) {
+  constexpr int MS = D + 4;  // mean row in LDS: the four groups' rows start in different banks
+  const int i = lane & 15;
+  float* mean = sh + (lane >> 4) * MS;
+  const int c0 = j * p.radix;
+  const int cn = p.n - c0 < p.radix ? p.n - c0 : p.radix;  // valid children
+  const int ncand = cn * p.P;
+  const uint16_t* child = static_cast<const uint16_t*>(p.child) + ((s * p.n + c0) * p.P) * (int64_t)D;
+  const uint16_t* mine = child + (int64_t)(i < ncand ? i : ncand - 1) * D;
+  uint4 row[D / 8];
+#pragma unroll
+  for (int v = 0; v < D / 8; ++v) row[v] = *reinterpret_cast<const uint4*>(mine + 8 * v);
+  if (8 * i < D) {
+    constexpr int kAhead = 4;  // children's rows loaded together
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+    for (int b = 0; b < cn; b += kAhead) {
+      uint4 x[kAhead];
+#pragma unroll
+      for (int c = 0; c < kAhead; ++c) {
+        const int ch = b + c < cn ? b + c : cn - 1;
+        x[c] = *reinterpret_cast<const uint4*>(child + (int64_t)ch * p.P * D + 8 * i);
+      }
+#pragma unroll
+      for (int c = 0; c < kAhead; ++c)
+        if (b + c < cn) {
+          const uint32_t w[4] = {x[c].x, x[c].y, x[c].z, x[c].w};
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] = acc[e] + unpack1<F16>(e & 1 ? w[e / 2] >> 16 : w[e / 2] & 0xffffu);
+        }
+    }
+    const float den = (float)cn;
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = round16<F16>(round16<F16>(acc[e]) / den);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = pack2<F16>(acc[2 * e], acc[2 * e + 1]);
+    *reinterpret_cast<float4*>(mean + 8 * i) = float4{acc[0], acc[1], acc[2], acc[3]};
+    *reinterpret_cast<float4*>(mean + 8 * i + 4) = float4{acc[4], acc[5], acc[6], acc[7]};
+    if (live)
+      *reinterpret_cast<uint4*>(static_cast<uint16_t*>(p.parent) + (s * p.m + j) * (int64_t)p.P * D + 8 * i) =
+          uint4{w[0], w[1], w[2], w[3]};
+  }
+  wave_sync();
+  float dist = 0.f;
+#pragma unroll
+  for (int v = 0; v < D / 8; ++v) {
+    const float4 m0 = *reinterpret_cast<const float4*>(mean + 8 * v);
+    const float4 m1 = *reinterpret_cast<const float4*>(mean + 8 * v + 4);
+    const float mv[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+    const uint32_t w[4] = {row[v].x, row[v].y, row[v].z, row[v].w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float df = unpack1<F16>(e & 1 ? w[e / 2] >> 16 : w[e / 2] & 0xffffu) - mv[e];
+      dist = dist + df * df;
+    }
+  }
+  // Distance order (NaN farthest, +0 and -0 equal) as an unsigned image, 0
+  // for lanes without a candidate; ties to the lower candidate.
+  const uint32_t key = i < ncand ? score_order(dist) : 0u;
+  int rank = 0;
+  auto count = [&](auto rc) {
+    constexpr int r = decltype(rc)::value;  // row_ror:r: lane i sees lane (i - r) mod 16
+    const uint32_t ko = (uint32_t)__builtin_amdgcn_mov_dpp((int)key, 0x120 + r, 0xf, 0xf, true);
+    rank += ko > key || (ko == key && ((i - r) & 15) < i) ? 1 : 0;
+  };
+  for_each_index(count, std::make_integer_sequence<int, 15>{});
+  if (live && i < ncand && rank < p.P - 1) {
+    uint16_t* out = static_cast<uint16_t*>(p.parent) + ((s * p.m + j) * (int64_t)p.P + 1 + rank) * D;
+#pragma unroll
+    for (int v = 0; v < D / 8; ++v) *reinterpret_cast<uint4*>(out + 8 * v) = row[v];
+  }
+  wave_sync();  // the mean rows are free for the next parents
+}
+
+// One wide level: a wavefront per four parents (counted over all slabs).
+template <bool F16, int D>
+__global__ __launch_bounds__(64) void tree_merge_four_kernel(const MergeParams p) {
+  __shared__ __attribute__((aligned(16))) float sh[4 * (D + 4)];
+  const int64_t total = p.S * p.m;
+  int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 4);
+  const bool live = g < total;
+  g = live ? g : total - 1;
+  const int64_t s = g / p.m;
+  merge_four<F16, D>(p, s, (int)(g - s * p.m), live, threadIdx.x, sh);
+}
+
 // One wavefront per (slab, parent node).
 __global__ __launch_bounds__(64) void tree_merge_kernel(const MergeParams p) {
   extern __shared__ float sh[];
@@ -226,6 +339,45 @@ __global__ __launch_bounds__(64 * kTopWaves) void tree_merge_top_kernel(const Me
     for (int j = wave; j < p.m; j += nw) merge_parent(p, s, j, lane, mine);
     __syncthreads();
   }
+}
+
+// The narrow levels with four parents per wavefront (merge_four).
+template <bool F16, int D>
+__global__ __launch_bounds__(64 * kTopWaves) void tree_merge_four_top_kernel(const MergeTopParams t) {
+  __shared__ __attribute__((aligned(16))) float sh[kTopWaves * 4 * (D + 4)];
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), nw = (int)(blockDim.x >> 6);
+  const int lane = threadIdx.x & 63;
+  for (int v = 0; v < t.levels; ++v) {
+    MergeParams p = t.p;
+    p.child = t.lvl[v];
+    p.parent = t.lvl[v + 1];
+    p.n = t.n[v];
+    p.m = t.n[v + 1];
+    for (int j0 = 4 * wave; j0 < p.m; j0 += 4 * nw) {
+      const int j = j0 + (lane >> 4);
+      merge_four<F16, D>(p, blockIdx.x, j < p.m ? j : p.m - 1, j < p.m, lane, sh + wave * 4 * (D + 4));
+    }
+    __syncthreads();
+  }
+}
+
+// Calls go(F16, D) with the kernels' template arguments when merge_four
+// covers the shape (its comment states it); false otherwise.
+template <typename Go>
+bool merge_four_applies(int dtype, int64_t P, int64_t D, int64_t radix, bool aligned, Go go) {
+  if (!aligned || radix * P > 16 || (D != 64 && D != 128)) return false;
+  using T = std::true_type;
+  using F = std::false_type;
+  if (dtype == SPRUCE_DTYPE_BF16) {
+    if (D == 64) go(F{}, std::integral_constant<int, 64>{});
+    else go(F{}, std::integral_constant<int, 128>{});
+  } else if (dtype == SPRUCE_DTYPE_F16) {
+    if (D == 64) go(T{}, std::integral_constant<int, 64>{});
+    else go(T{}, std::integral_constant<int, 128>{});
+  } else {
+    return false;
+  }
+  return true;
 }
 
 struct ScoreParams2 {
@@ -725,6 +877,11 @@ extern "C" int spruce_tree_merge_level(const void* child, int64_t S, int64_t n, 
   p.dtype = dtype;
   p.vec = (D % 8 == 0 && ((uintptr_t)child % 16) == 0) ? 1 : 0;
   SPRUCE_REQUIRE(S * p.m < ((int64_t)1 << 31), "too many parent nodes");
+  if (merge_four_applies(dtype, P, D, radix, ((uintptr_t)child | (uintptr_t)parent) % 16 == 0, [&](auto f16, auto dim) {
+        hipLaunchKernelGGL((tree_merge_four_kernel<decltype(f16)::value, decltype(dim)::value>),
+                           dim3((unsigned)((S * p.m + 3) / 4)), dim3(64), 0, (hipStream_t)stream, p);
+      }))
+    return check_launch("tree_merge_four_kernel");
   const size_t lds = ((size_t)radix * P * (D + 4) + D) * sizeof(float);
   SPRUCE_REQUIRE(lds <= 65536, "radix * P * D too large for one workgroup's LDS (%zu bytes)", lds);
   hipLaunchKernelGGL(tree_merge_kernel, dim3((unsigned)(S * p.m)), dim3(64), lds, (hipStream_t)stream, p);
@@ -748,6 +905,9 @@ extern "C" int spruce_tree_merge_levels(const void* child, int64_t S, int64_t n,
   SPRUCE_REQUIRE(dtype == SPRUCE_DTYPE_BF16 || dtype == SPRUCE_DTYPE_F16 || dtype == SPRUCE_DTYPE_F32,
                  "unsupported dtype code %d", dtype);
   for (int v = 0; v < levels; ++v) SPRUCE_REQUIRE(parents[v], "parent level %d is a null pointer", v);
+  bool aligned = (uintptr_t)child % 16 == 0;
+  for (int v = 0; v < levels; ++v) aligned = aligned && (uintptr_t)parents[v] % 16 == 0;
+  const bool four = merge_four_applies(dtype, P, D, radix, aligned, [](auto, auto) {});
   const int64_t wave_lds = radix * P * (D + 4) + D;
   int64_t waves = wave_lds > 0 ? 65536 / (wave_lds * (int64_t)sizeof(float)) : 0;
   waves = waves > kTopWaves ? kTopWaves : waves;
@@ -755,8 +915,9 @@ extern "C" int spruce_tree_merge_levels(const void* child, int64_t S, int64_t n,
   const void* cur = child;
   for (int v = 0; v < levels; ++v) {
     const int64_t m = (cur_n + radix - 1) / radix;
-    if (m <= waves) {
-      // Every remaining level has at most one parent per wavefront.
+    // One workgroup per slab forms the remaining levels once its wavefronts
+    // take a level's parents in one go.
+    if (m <= (four ? 4 * kTopWaves : waves)) {
       MergeTopParams t{};
       t.p.S = S;
       t.p.P = (int)P;
@@ -770,6 +931,14 @@ extern "C" int spruce_tree_merge_levels(const void* child, int64_t S, int64_t n,
         t.n[u + 1] = (t.n[u] + (int)radix - 1) / (int)radix;
         t.lvl[u + 1] = parents[v + u];
         t.vec[u] = (D % 8 == 0 && ((uintptr_t)t.lvl[u] % 16) == 0) ? 1 : 0;
+      }
+      if (four) {
+        const unsigned w = (unsigned)((m + 3) / 4);
+        merge_four_applies(dtype, P, D, radix, true, [&](auto f16, auto dim) {
+          hipLaunchKernelGGL((tree_merge_four_top_kernel<decltype(f16)::value, decltype(dim)::value>),
+                             dim3((unsigned)S), dim3(64 * w), 0, (hipStream_t)stream, t);
+        });
+        return check_launch("tree_merge_four_top_kernel");
       }
       t.wave_lds = (int)wave_lds;
       const size_t lds = (size_t)waves * wave_lds * sizeof(float);
