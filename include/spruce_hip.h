@@ -252,6 +252,14 @@ int spruce_mask_key_validity(const void* mask, const int64_t ms[4], int64_t Hm, 
                              uint8_t* valid, int32_t* flags, void* stream);
 
 /*
+ * Sets flag[0] when one of the `rows` contiguous int32 rows of K block ids
+ * lists no block (every entry negative); otherwise leaves it.  Serves the
+ * empty-row check of sparse_prefill_attention_forward
+ * (sparse/attention.py:192-199 in the reference).
+ */
+int spruce_empty_rows(const int32_t* ids, int64_t rows, int64_t K, int32_t* flag, void* stream);
+
+/*
  * Residual-tree frontiers.  Replaces build_residual_summary_nodes /
  * residual_frontier_for_row (interfaces/residual_summaries.py:119-222): for
  * each row (b, l, g, q) of selected [B, L, G, Qb, K] int32 (element strides

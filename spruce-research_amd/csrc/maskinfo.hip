@@ -130,10 +130,29 @@ __global__ __launch_bounds__(256) void mask_key_validity_kernel(const MaskParams
   }
 }
 
+// Rows with no listed block (every entry negative) among `rows` contiguous
+// rows of K: a thread per row, one read of the lists.
+__global__ __launch_bounds__(256) void empty_rows_kernel(const int32_t* __restrict__ ids, int64_t rows, int64_t K,
+                                                         int32_t* flag) {
+  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (r >= rows) return;
+  bool listed = false;
+  for (int64_t k = 0; k < K && !listed; ++k) listed = ids[r * K + k] >= 0;
+  if (!listed) *flag = 1;
+}
+
 }  // namespace
 }  // namespace spruce
 
 using namespace spruce;
+
+extern "C" int spruce_empty_rows(const int32_t* ids, int64_t rows, int64_t K, int32_t* flag, void* stream) {
+  SPRUCE_REQUIRE(ids && flag, "ids and flag must be non-null");
+  SPRUCE_REQUIRE(rows >= 1 && K >= 1 && K < ((int64_t)1 << 31) && rows < ((int64_t)1 << 38), "invalid list shape");
+  hipLaunchKernelGGL(empty_rows_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, (hipStream_t)stream, ids,
+                     rows, K, flag);
+  return check_launch("empty_rows_kernel");
+}
 
 extern "C" int spruce_mask_key_validity(const void* mask, const int64_t ms[4], int64_t Hm, int mask_dtype, int64_t B,
                                         int64_t T, uint8_t* valid, int32_t* flags, void* stream) {

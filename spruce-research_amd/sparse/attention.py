@@ -98,7 +98,29 @@ def _validate_inputs(query, key, value, selected_blocks, block_size, layer_idx, 
 _EMPTY_ROWS = [None]   # (weakref to selected_blocks, its version, {layer: first empty row})
 
 
-def _empty_rows(selected_blocks: torch.Tensor) -> dict:
+def _known_empty_rows(selected_blocks: torch.Tensor) -> Optional[dict]:
+    """The kept answer of ``_empty_rows`` for this tensor, or None."""
+    last = _EMPTY_ROWS[0]
+    if (not selected_blocks.is_inference() and last is not None and last[0]() is selected_blocks
+            and last[1] == selected_blocks._version):
+        return last[2]
+    return None
+
+
+def _launch_empty_check(selected_blocks: torch.Tensor, flags: torch.Tensor) -> bool:
+    """Issues the kernel that sets ``flags[2]`` when some row lists no block;
+    False where it does not read the tensor (host, other dtype, strides)."""
+    s = selected_blocks
+    if not (s.is_cuda and s.device == flags.device and s.dtype == torch.int32 and s.is_contiguous() and s.numel()):
+        return False
+    with spruce_hip.on_device(s.device):
+        rc = spruce_hip.lib().spruce_empty_rows(spruce_hip.ptr(s), s.numel() // s.shape[-1], s.shape[-1],
+                                                spruce_hip.ptr(flags) + 8, spruce_hip.stream_of(s))
+    spruce_hip.check(rc, "spruce_empty_rows")
+    return True
+
+
+def _empty_rows(selected_blocks: torch.Tensor, none_empty: bool = False) -> dict:
     """{layer: (batch, kv_head, query_block) of its first row with no listed
     block}, for every layer of ``selected_blocks`` at once.  Reading the
     answer back waits for the GPU, so it is done once per selected_blocks
@@ -106,18 +128,18 @@ def _empty_rows(selected_blocks: torch.Tensor) -> dict:
     and unmodified, instead of stalling the host at every layer.  Tensors
     made under ``torch.inference_mode`` have no version counter, so an
     in-place change to them could not be seen: they are checked at every
-    call."""
-    tracked = not selected_blocks.is_inference()
-    last = _EMPTY_ROWS[0]
-    if (tracked and last is not None and last[0]() is selected_blocks
-            and last[1] == selected_blocks._version):
-        return last[2]
-    empty = ~(selected_blocks >= 0).any(dim=-1)        # [B, L, G, Qb]
+    call.  ``none_empty``: a check of this call found no such row."""
+    known = _known_empty_rows(selected_blocks)
+    if known is not None:
+        return known
     found = {}
-    if bool(empty.any()):
-        for b, layer, g, qb in torch.nonzero(empty).tolist():
-            found.setdefault(layer, (b, g, qb))
-    if tracked:
+    if not none_empty:
+        flags = torch.zeros(3, device=selected_blocks.device, dtype=torch.int32)
+        if not _launch_empty_check(selected_blocks, flags) or int(flags[2]):
+            empty = ~(selected_blocks >= 0).any(dim=-1)        # [B, L, G, Qb]
+            for b, layer, g, qb in torch.nonzero(empty).tolist():
+                found.setdefault(layer, (b, g, qb))
+    if not selected_blocks.is_inference():
         _EMPTY_ROWS[0] = (weakref.ref(selected_blocks), selected_blocks._version, found)
     return found
 
@@ -176,24 +198,27 @@ def _key_validity(attention_mask: torch.Tensor, batch: int, seq_len: int) -> Opt
 _MASK_CODES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2, torch.bool: 3}
 
 
-def _key_validity_and_padding(attention_mask: torch.Tensor, batch: int, seq_len: int) -> tuple:
-    """(``_key_validity``, whether some key is padding) of a mask: on the GPU
-    one launch that reads the mask once and one read back of its two flags;
-    masks the kernel does not read (other dtypes, strided rows, host tensors)
-    take the tensor operations above."""
+def _key_validity_and_padding(attention_mask: torch.Tensor, batch: int, seq_len: int,
+                              selected_blocks: Optional[torch.Tensor] = None) -> tuple:
+    """(``_key_validity``, whether some key is padding, whether the lists of
+    ``selected_blocks`` were found to have no empty row) of a mask: on the
+    GPU one launch that reads the mask once, one that reads the lists, and
+    one read back of their flags; masks the kernel does not read (other
+    dtypes, strided rows, host tensors) take the tensor operations above."""
     m = attention_mask
     if not (m.is_cuda and m.dtype in _MASK_CODES and m.stride(-1) == 1 and m.numel()):
         valid = _key_validity(m, batch, seq_len)
-        return valid, valid is not None and not bool(valid.all())
+        return valid, valid is not None and not bool(valid.all()), False
     valid = torch.empty((batch, seq_len), device=m.device, dtype=torch.bool)
-    flags = torch.zeros(2, device=m.device, dtype=torch.int32)
+    flags = torch.zeros(3, device=m.device, dtype=torch.int32)
     with spruce_hip.on_device(m.device):
         rc = spruce_hip.lib().spruce_mask_key_validity(
             spruce_hip.ptr(m), spruce_hip.strides(m), m.shape[1], _MASK_CODES[m.dtype], batch, seq_len,
             spruce_hip.ptr(valid), spruce_hip.ptr(flags), spruce_hip.stream_of(m))
     spruce_hip.check(rc, "spruce_mask_key_validity")
-    other, padded = flags.tolist()
-    return (None, False) if other else (valid, bool(padded))
+    checked = selected_blocks is not None and _launch_empty_check(selected_blocks, flags)
+    other, padded, empty = flags.tolist()
+    return (None, False, checked and not empty) if other else (valid, bool(padded), checked and not empty)
 
 
 def sparse_prefill_attention_forward(
@@ -245,9 +270,12 @@ def sparse_prefill_attention_forward(
                 validate_selected=not validate_selected_blocks_input)
     key_valid = None
     general_mask = None
+    none_empty = False
     if attention_mask is not None:
         _check_mask_shape(attention_mask, query.shape[0], query.shape[1], query.shape[-2])
-        key_valid, padded = _key_validity_and_padding(attention_mask, query.shape[0], query.shape[-2])
+        unchecked = selected_blocks if _known_empty_rows(selected_blocks) is None else None
+        key_valid, padded, none_empty = _key_validity_and_padding(
+            attention_mask, query.shape[0], query.shape[-2], unchecked)
         if key_valid is None:
             if residual_summaries:
                 raise ValueError(
@@ -260,7 +288,7 @@ def sparse_prefill_attention_forward(
         raise ValueError("the HIP sparse-prefill kernel requires block_size=64")
     indices = selected_blocks[:, layer_idx].to(device=query.device, dtype=torch.int32).contiguous()
     # The reference raises on a row with no selected block (sparse/attention.py:192-199).
-    empty_row = _empty_rows(selected_blocks).get(layer_idx)
+    empty_row = _empty_rows(selected_blocks, none_empty).get(layer_idx)
     if empty_row is not None:
         b, g, qb = empty_row
         raise ValueError(

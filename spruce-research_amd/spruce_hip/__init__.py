@@ -91,6 +91,7 @@ _SIGNATURES = {
         _p, _STRIDES, _i64, _p, _p, _p, ctypes.c_int, _i64, _i64,
         _i64, _i64, _i64, _i64, _i64, ctypes.c_float, ctypes.c_int, ctypes.c_int,
         _p, _STRIDES, _p],
+    "spruce_empty_rows": [_p, _i64, _i64, _p, _p],
     "spruce_mask_key_validity": [_p, _STRIDES, _i64, ctypes.c_int, _i64, _i64, _p, _p, _p],
     "spruce_sparse_prefill_index_amask": [
         _p, _STRIDES, _p, _STRIDES, _p, _STRIDES, _p, _STRIDES, _i64, _p, _STRIDES, _i64, _i64, _i64,

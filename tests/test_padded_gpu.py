@@ -231,7 +231,45 @@ def test_mask_reduction_kernel_equals_the_tensor_operations(dtype):
             wide = torch.empty(m.shape[:3] + (T + 3,), dtype=dtype)
             wide[..., 3:] = m
             for dev in (m.to(DEV), wide.to(DEV)[..., 3:], m.transpose(2, 3).contiguous().to(DEV).transpose(2, 3)):
-                got, padded = _key_validity_and_padding(dev, B, T)
+                got, padded, _ = _key_validity_and_padding(dev, B, T)
                 assert (got is None) == (want is None)
                 if want is not None:
                     assert torch.equal(got.cpu(), want) and padded == (not bool(want.all()))
+
+
+def test_empty_row_check_equals_the_tensor_operations():
+    # The list check beside the mask's flags, and alone: no empty row, one in
+    # the first, middle or last row of a layer, rows led by padding, single
+    # rows, host and strided tensors, and after an in-place change.
+    from sparse import attention as sa
+    gen = torch.Generator().manual_seed(9)
+    mask, _ = torch.ones(1, 1, 8, 8, dtype=torch.bool).tril().to(DEV), None
+    for shape in ((1, 1, 1, 1, 1), (2, 3, 2, 5, 4), (1, 4, 4, 301, 18)):
+        base = torch.randint(0, 5, shape, generator=gen, dtype=torch.int32)
+        base[..., : shape[-1] // 2] = -1
+        rows = base.view(-1, shape[-1])
+        for empty in (None, 0, len(rows) // 2, len(rows) - 1):
+            lists = base.clone()
+            if empty is not None:
+                lists.view(-1, shape[-1])[empty] = -1
+            want = {}
+            for b, layer, g, qb in torch.nonzero(~(lists >= 0).any(-1)).tolist():
+                want.setdefault(layer, (b, g, qb))
+            wide = torch.full(shape[:-1] + (shape[-1] + 1,), -1, dtype=torch.int32)
+            wide[..., :-1] = lists
+            for s in (lists.to(DEV), wide.to(DEV)[..., :-1], lists, lists.long().to(DEV)):
+                sa._EMPTY_ROWS[0] = None
+                assert sa._empty_rows(s) == want
+                assert sa._known_empty_rows(s) == want
+                sa._EMPTY_ROWS[0] = None
+                found = sa._key_validity_and_padding(mask, 1, 8, s)[2]
+                direct = s.is_cuda and s.dtype == torch.int32 and s.is_contiguous()
+                assert found == (direct and not want)
+                sa._EMPTY_ROWS[0] = None
+                s[0, 0, 0, 0] = -1
+                assert 0 in sa._empty_rows(s)
+                with torch.inference_mode():
+                    inferred = s.clone()
+                    assert 0 in sa._empty_rows(inferred)
+                    inferred.fill_(0)
+                    assert sa._empty_rows(inferred) == {}
