@@ -454,3 +454,22 @@ def test_projection_of_layers_equals_each_layer(dtype, L, S, nodes, Pk, D, P):
         assert torch.equal(gate.project_queries(levels[0]), want)
         odd = torch.empty(levels[0].numel() + 1, dtype=dtype, device=DEV)[1:].view(levels[0].shape).copy_(levels[0])
         assert torch.equal(gate.project_queries(odd), want)   # not 16-byte aligned: the general kernels
+
+
+@pytest.mark.parametrize("Kb", [1, 63, 64, 65, 255, 256, 257, 512, 513, 1024])
+def test_topk_slots_per_lane(Kb):
+    # Rows held in 4, 8 or 16 slots a lane: the widths where the slot count
+    # changes, with ties, both zeros and infinities, k below and above
+    # the 64-candidate search's reach and above the row.
+    gen = torch.Generator().manual_seed(Kb)
+    s = torch.randn(2, Kb, Kb, generator=gen)
+    s[0, :, ::3] = s[0, :, :1].clone()
+    s[1, :, ::5] = 0.0
+    s[1, :, 1::7] = -0.0
+    if Kb > 8:
+        s[1, Kb - 1, 3] = float("inf")
+        s[1, Kb - 2, 5] = float("-inf")
+    for k in (1, 8, 64, 65, 100):
+        print(f"topk Kb={Kb} k={k}", flush=True)
+        got = causal_topk_blocks(s.to(DEV), k).cpu().numpy()
+        np.testing.assert_array_equal(got, osel.topk(s.numpy(), k))
