@@ -266,9 +266,9 @@ def main():
         "tflops": round(flops1 / (m1 * 1e-3) / 1e12, 2),
         "frac_bf16_peak": round(flops1 / (m1 * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, 4),
         "selected_head_blocks": sel1, "flop": flops1, "input_dtype": "fp32",
-        "note": "128 (KV head, query block) rows split into 2 four-wave parts: 256 workgroups, "
-                "one per CU, each over a few blocks, so this small case is launch- and "
-                "latency-bound",
+        "note": "128 (KV head, query block) rows split into 2 four-tile parts: 256 workgroups, "
+                "one per CU, each over a few blocks, so this small case is bound by the longest "
+                "row's chain of blocks",
     }
     if not args.no_cpu:
         configs["cfg1_4k_block_mask_fp32"]["cpu_baseline"] = cpu_baseline_cfg1(q1, k1, v1, mask1, flops1)
@@ -370,9 +370,8 @@ def main():
                 "radix": 2, "k_selected": beam + 2,
                 "stages": stages,
                 "note": ("floor = sum over stages of max(bytes / 8 TB/s, flop / 157.3 TFLOP/s fp32); "
-                         "traverse is the dominant kernel (tree_traverse_kernel, fp32 VALU dot products; "
-                         "157.3 TFLOP/s assumes packed FP32, which this build does not emit, so 78.6 is "
-                         "its VALU ceiling)"),
+                         "traverse is the dominant kernel (tree_traverse_kernel, fp32 dot products on the "
+                         "matrix cores)"),
             }
             del qf, kf, levels, qp, kp, ids
         del q5, k5, v5

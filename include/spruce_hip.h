@@ -437,10 +437,11 @@ int spruce_tree_merge_level(const void* child, int64_t S, int64_t n, int64_t P, 
  *   parents    host array of `levels` device pointers; parents[v] is level
  *              v + 1 above the child, [S, n_{v+1}, P, D] contiguous, with
  *              n_{v+1} = ceil(n_v / radix) and n_0 = n.
- * Wide levels get one launch each (one wavefront per parent); once a level
- * has no more parents than fit as wavefronts of one workgroup in 64 KB of
- * LDS (at most 16), it and every level above it share one launch, one
- * workgroup per slab.  1 <= levels <= 32; other limits as
+ * Wide levels get one launch each.  Narrow levels share one launch, one
+ * workgroup per slab: from the first level of at most 64 parents where four
+ * parents share a wavefront (16-bit nodes, D 64 or 128, radix*P <= 16, 16-byte
+ * aligned levels), else from the first whose parents fit as wavefronts of one
+ * workgroup in 64 KB of LDS (at most 16).  1 <= levels <= 32; other limits as
  * spruce_tree_merge_level.
  */
 int spruce_tree_merge_levels(const void* child, int64_t S, int64_t n, int64_t P, int64_t D, int64_t radix,

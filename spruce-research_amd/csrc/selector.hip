@@ -1022,8 +1022,8 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
       }
 }
 
-// The same scores for prototype counts whose tiles do not fit in LDS (e.g.
-// 8 x 8 prototypes of 128 dims): one thread per score, operands read through
+// The same scores for prototype counts that are not 1, 2, 4 or 8 and whose
+// tiles do not fit in LDS (e.g. 12 x 12 prototypes of 128 dims): one thread per score, operands read through
 // the cache, identical operation order.
 __global__ __launch_bounds__(256) void gate_scores_direct_kernel(const ScoreParams p, int64_t total) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;

@@ -1,8 +1,10 @@
 // Tree selector on gfx950: the key-axis prototype tree and its top-down beam
 // traversal, the deployed route producer.
 //
-//   tree_merge_kernel     one parent level of build_key_tree
-//   tree_merge_top_kernel the narrow levels near the root, in one launch
+//   tree_merge_kernel, tree_merge_four_kernel
+//                         one parent level of build_key_tree
+//   tree_merge_top_kernel, tree_merge_four_top_kernel
+//                         the narrow levels near the root, in one launch
 //                         (selector/tree.py:79-145, _merge_level_prototypes)
 //   tree_traverse_kernel  traverse_to_leaf_ids
 //                         (scripts/eval_tree_traversal.py:59-113)
