@@ -843,6 +843,11 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_max(float x) {
   return fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true)));
 }
+template <int CTRL>
+__device__ __forceinline__ int dpp_min(int x) {
+  const int y = __builtin_amdgcn_mov_dpp(x, CTRL, 0xf, 0xf, true);
+  return y < x ? y : x;
+}
 
 // The scores above for 1, 2, 4 or 8 prototypes a side, as one matrix product
 // of prototype rows: a workgroup of 2 x 2 waves covers 64 RA query rows x 128
@@ -850,8 +855,10 @@ __device__ __forceinline__ float dpp_max(float x) {
 // per (query block, key block): the PQ rows of a query block are registers of
 // one lane (and its other half for PQ = 8), the PK columns neighbouring lanes.
 // fmaxf drops NaN as "replace when strictly larger" does, except for the
-// first pair, which the writing lane holds itself and keeps if it is NaN; a
-// maximum of exactly zero may take either sign.
+// first pair, which the writing lane holds itself and keeps if it is NaN.
+// Where the maximum is zero that rule keeps the first zero's sign, and fmaxf
+// need not: a wavefront with such a score and a negative zero among its
+// products looks for that pair in a second pass (the test for it: 0.3%).
 //
 // Bound: fp32 MFMA issue (busy 68% of the cycles; three waves a SIMD, the
 // rest is each tile's first loads and its reduction).  8 x 8 prototypes,
@@ -1000,26 +1007,71 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
     return;
   }
   constexpr int GS = PQ < 4 ? PQ : 4;  // rows of one query block among a lane's four consecutive ones
+  bool zero = false;
+  auto each_group = [&](int lane, auto f) {
 #pragma unroll
-  for (int a = 0; a < RA; ++a)
+    for (int a = 0; a < RA; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+      for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int r0 = 0; r0 < 16; r0 += GS) {
-        const float first = acc[a][b][r0];
-        float m = first;
+        for (int r0 = 0; r0 < 16; r0 += GS) {
+          float m = acc[a][b][r0];
 #pragma unroll
-        for (int r = 1; r < GS; ++r) m = fmaxf(m, acc[a][b][r0 + r]);
-        if constexpr (PQ == 8) m = half_max(m);
-        if constexpr (PK >= 2) m = dpp_max<0xB1>(m);   // quad_perm [1, 0, 3, 2]
-        if constexpr (PK >= 4) m = dpp_max<0x4E>(m);   // quad_perm [2, 3, 0, 1]
-        if constexpr (PK >= 8) m = dpp_max<0x141>(m);  // row_half_mirror
-        if (first != first) m = first;
-        const int row = 32 * a + 8 * (r0 / 4) + (PQ == 8 ? 0 : 4 * (lane >> 5)) + r0 % 4;
-        const int i = iw + row / PQ, j = jw + (32 * b + (lane & 31)) / PK;
-        if (lane % PK == 0 && (PQ < 8 || lane < 32) && i < p.Qb && j < p.Kb)
-          out[(int64_t)i * p.Kb + j] = (!p.causal || j <= i) ? m / p.div : -INFINITY;
+          for (int r = 1; r < GS; ++r) m = fmaxf(m, acc[a][b][r0 + r]);
+          if constexpr (PQ == 8) m = half_max(m);
+          if constexpr (PK >= 2) m = dpp_max<0xB1>(m);   // quad_perm [1, 0, 3, 2]
+          if constexpr (PK >= 4) m = dpp_max<0x4E>(m);   // quad_perm [2, 3, 0, 1]
+          if constexpr (PK >= 8) m = dpp_max<0x141>(m);  // row_half_mirror
+          const int row = 32 * a + 8 * (r0 / 4) + (PQ == 8 ? 0 : 4 * (lane >> 5)) + r0 % 4;
+          const int i = iw + row / PQ, j = jw + (32 * b + (lane & 31)) / PK;
+          const bool writes = lane % PK == 0 && (PQ < 8 || lane < 32) && i < p.Qb && j < p.Kb;
+          f(acc[a][b], r0, m, writes, i, j);
+        }
+  };
+  each_group(lane, [&](const f32x16_t& c, int r0, float m, bool writes, int i, int j) {
+    zero |= m == 0.f;
+    const float first = c[r0];
+    if (first != first) m = first;
+    if (writes) out[(int64_t)i * p.Kb + j] = (!p.causal || j <= i) ? m / p.div : -INFINITY;
+  });
+  if constexpr (PQ * PK > 1) {
+    if (__ballot(zero) == 0) return;
+    // With no negative zero among the products every zero score is right.
+    bool negative = false;
+#pragma unroll
+    for (int a = 0; a < RA; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float x = acc[a][b][r];
+          negative |= __builtin_bit_cast(uint32_t, x) == 0x80000000u;
+        }
+    if (__ballot(negative) == 0) return;
+    // Zero scores again: the place of the first zero in pair order and its
+    // sign.  (The lane is hidden from the compiler, which would keep every
+    // store's mask from the pass above in scalar registers.)
+    int again = lane;
+    asm volatile("" : "+v"(again));
+    each_group(again, [&](const f32x16_t& c, int r0, float m, bool writes, int i, int j) {
+      int at = 2 * PQ * PK;  // 2 place + sign
+#pragma unroll
+      for (int r = GS - 1; r >= 0; --r) {
+        const int place = ((PQ == 8 ? 4 * (lane >> 5) : 0) + r) * PK + lane % PK;
+        const float x = c[r0 + r];
+        if (x == 0.f) at = 2 * place + (__builtin_bit_cast(int, x) < 0 ? 1 : 0);
       }
+      if constexpr (PQ == 8) {
+        const int other = __shfl_xor(at, 32);
+        at = other < at ? other : at;
+      }
+      if constexpr (PK >= 2) at = dpp_min<0xB1>(at);
+      if constexpr (PK >= 4) at = dpp_min<0x4E>(at);
+      if constexpr (PK >= 8) at = dpp_min<0x141>(at);
+      if (writes && m == 0.f && c[r0] == c[r0] && (!p.causal || j <= i))
+        out[(int64_t)i * p.Kb + j] = (at & 1 ? -0.f : 0.f) / p.div;
+    });
+  }
 }
 
 // The same scores for prototype counts that are not 1, 2, 4 or 8 and whose

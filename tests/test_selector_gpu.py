@@ -429,6 +429,32 @@ def test_matrix_scores_are_bit_exact(Pq, Pk):
             np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("Pq", [1, 2, 4, 8])
+@pytest.mark.parametrize("Pk", [1, 2, 4, 8])
+def test_matrix_scores_keep_the_sign_of_zero(Pq, Pk):
+    # Pairs of exact zeros and of products that underflow to either zero: the
+    # first zero of a maximum of zero stays (later pairs are not strictly
+    # larger), so its sign is the oracle's; NaN pairs among them stay out.
+    gen = torch.Generator().manual_seed(40 * Pq + Pk)
+    zeros = torch.tensor([0.0, -0.0, 1e-30, -1e-30])
+    negative = 0
+    for Qb, Kb, P in ((70, 70, 4), (33, 150, 12), (300, 300, 4)):
+        qp = zeros[torch.randint(0, 4, (2, Qb, Pq, P), generator=gen)]
+        kp = zeros[torch.randint(0, 4, (2, Kb, Pk, P), generator=gen)]
+        if P == 4:   # pairs below zero too, so that the first zero is not the first pair
+            qp[1, :, :, 0] = torch.randn(Qb, Pq, generator=gen).sign()
+            kp[1, :, :, 0] = torch.randn(Kb, Pk, generator=gen).sign()
+            kp[0, 5, -1, 1] = float("nan")
+        for causal in (False, True):
+            got = _np(gate_scores(qp.to(DEV), kp.to(DEV), causal=causal))
+            want = osel.scores(qp.numpy(), kp.numpy(), causal=causal)
+            np.testing.assert_array_equal(got, want)
+            zero = want == 0
+            np.testing.assert_array_equal(np.signbit(got[zero]), np.signbit(want[zero]))
+            negative += int(np.signbit(want[zero]).sum())
+    assert negative > 100
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("L,S,nodes,Pk,D,P", [
     (1, 1, [1], 1, 4, 4), (3, 2, [37, 19, 1], 8, 36, 64), (2, 1, [70], 4, 128, 132), (2, 3, [1500, 750, 5], 8, 32, 260)])
