@@ -839,14 +839,32 @@ __global__ __launch_bounds__(256) void gate_scores_kernel(const ScoreParams p) {
   }
 }
 
+// One score, pair by pair, its operands read through the cache.
+__device__ __forceinline__ float score_in_order(const ScoreParams& p, int64_t bg, int i, int j) {
+  const float* qrow = p.qp + (bg * p.Qb + i) * (int64_t)p.Pq * p.P;
+  const float* krow = p.kp + (bg * p.Kb + j) * (int64_t)p.Pk * p.P;
+  float best = 0.f;
+  for (int a = 0; a < p.Pq; ++a)
+    for (int c = 0; c < p.Pk; ++c) {
+      const float4* x = reinterpret_cast<const float4*>(qrow + a * p.P);
+      const float4* y = reinterpret_cast<const float4*>(krow + c * p.P);
+      float acc = 0.f;
+#pragma unroll 4
+      for (int e = 0; e < p.P / 4; ++e) {
+        const float4 xv = x[e], yv = y[e];
+        acc = __builtin_fmaf(xv.x, yv.x, acc);
+        acc = __builtin_fmaf(xv.y, yv.y, acc);
+        acc = __builtin_fmaf(xv.z, yv.z, acc);
+        acc = __builtin_fmaf(xv.w, yv.w, acc);
+      }
+      best = (a == 0 && c == 0) ? acc : (acc > best ? acc : best);
+    }
+  return best / p.div;
+}
+
 template <int CTRL>
 __device__ __forceinline__ float dpp_max(float x) {
   return fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true)));
-}
-template <int CTRL>
-__device__ __forceinline__ int dpp_min(int x) {
-  const int y = __builtin_amdgcn_mov_dpp(x, CTRL, 0xf, 0xf, true);
-  return y < x ? y : x;
 }
 
 // The scores above for 1, 2, 4 or 8 prototypes a side, as one matrix product
@@ -858,7 +876,7 @@ __device__ __forceinline__ int dpp_min(int x) {
 // first pair, which the writing lane holds itself and keeps if it is NaN.
 // Where the maximum is zero that rule keeps the first zero's sign, and fmaxf
 // need not: a wavefront with such a score and a negative zero among its
-// products looks for that pair in a second pass (the test for it: 0.3%).
+// products (they underflowed) scores its pairs again in order.
 //
 // Bound: fp32 MFMA issue (busy 68% of the cycles; three waves a SIMD, the
 // rest is each tile's first loads and its reduction).  8 x 8 prototypes,
@@ -1007,37 +1025,30 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
     return;
   }
   constexpr int GS = PQ < 4 ? PQ : 4;  // rows of one query block among a lane's four consecutive ones
-  bool zero = false;
-  auto each_group = [&](int lane, auto f) {
+  bool zero = false, negative = false;
 #pragma unroll
-    for (int a = 0; a < RA; ++a)
+  for (int a = 0; a < RA; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int r0 = 0; r0 < 16; r0 += GS) {
-          float m = acc[a][b][r0];
+      for (int r0 = 0; r0 < 16; r0 += GS) {
+        const float first = acc[a][b][r0];
+        float m = first;
 #pragma unroll
-          for (int r = 1; r < GS; ++r) m = fmaxf(m, acc[a][b][r0 + r]);
-          if constexpr (PQ == 8) m = half_max(m);
-          if constexpr (PK >= 2) m = dpp_max<0xB1>(m);   // quad_perm [1, 0, 3, 2]
-          if constexpr (PK >= 4) m = dpp_max<0x4E>(m);   // quad_perm [2, 3, 0, 1]
-          if constexpr (PK >= 8) m = dpp_max<0x141>(m);  // row_half_mirror
-          const int row = 32 * a + 8 * (r0 / 4) + (PQ == 8 ? 0 : 4 * (lane >> 5)) + r0 % 4;
-          const int i = iw + row / PQ, j = jw + (32 * b + (lane & 31)) / PK;
-          const bool writes = lane % PK == 0 && (PQ < 8 || lane < 32) && i < p.Qb && j < p.Kb;
-          f(acc[a][b], r0, m, writes, i, j);
-        }
-  };
-  each_group(lane, [&](const f32x16_t& c, int r0, float m, bool writes, int i, int j) {
-    zero |= m == 0.f;
-    const float first = c[r0];
-    if (first != first) m = first;
-    if (writes) out[(int64_t)i * p.Kb + j] = (!p.causal || j <= i) ? m / p.div : -INFINITY;
-  });
+        for (int r = 1; r < GS; ++r) m = fmaxf(m, acc[a][b][r0 + r]);
+        if constexpr (PQ == 8) m = half_max(m);
+        if constexpr (PK >= 2) m = dpp_max<0xB1>(m);   // quad_perm [1, 0, 3, 2]
+        if constexpr (PK >= 4) m = dpp_max<0x4E>(m);   // quad_perm [2, 3, 0, 1]
+        if constexpr (PK >= 8) m = dpp_max<0x141>(m);  // row_half_mirror
+        zero |= m == 0.f;
+        if (first != first) m = first;
+        const int row = 32 * a + 8 * (r0 / 4) + (PQ == 8 ? 0 : 4 * (lane >> 5)) + r0 % 4;
+        const int i = iw + row / PQ, j = jw + (32 * b + (lane & 31)) / PK;
+        if (lane % PK == 0 && (PQ < 8 || lane < 32) && i < p.Qb && j < p.Kb)
+          out[(int64_t)i * p.Kb + j] = (!p.causal || j <= i) ? m / p.div : -INFINITY;
+      }
   if constexpr (PQ * PK > 1) {
     if (__ballot(zero) == 0) return;
-    // With no negative zero among the products every zero score is right.
-    bool negative = false;
 #pragma unroll
     for (int a = 0; a < RA; ++a)
 #pragma unroll
@@ -1048,29 +1059,11 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
           negative |= __builtin_bit_cast(uint32_t, x) == 0x80000000u;
         }
     if (__ballot(negative) == 0) return;
-    // Zero scores again: the place of the first zero in pair order and its
-    // sign.  (The lane is hidden from the compiler, which would keep every
-    // store's mask from the pass above in scalar registers.)
-    int again = lane;
-    asm volatile("" : "+v"(again));
-    each_group(again, [&](const f32x16_t& c, int r0, float m, bool writes, int i, int j) {
-      int at = 2 * PQ * PK;  // 2 place + sign
-#pragma unroll
-      for (int r = GS - 1; r >= 0; --r) {
-        const int place = ((PQ == 8 ? 4 * (lane >> 5) : 0) + r) * PK + lane % PK;
-        const float x = c[r0 + r];
-        if (x == 0.f) at = 2 * place + (__builtin_bit_cast(int, x) < 0 ? 1 : 0);
-      }
-      if constexpr (PQ == 8) {
-        const int other = __shfl_xor(at, 32);
-        at = other < at ? other : at;
-      }
-      if constexpr (PK >= 2) at = dpp_min<0xB1>(at);
-      if constexpr (PK >= 4) at = dpp_min<0x4E>(at);
-      if constexpr (PK >= 8) at = dpp_min<0x141>(at);
-      if (writes && m == 0.f && c[r0] == c[r0] && (!p.causal || j <= i))
-        out[(int64_t)i * p.Kb + j] = (at & 1 ? -0.f : 0.f) / p.div;
-    });
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // other lanes stored these scores above
+    for (int e = lane; e < (32 * RA / PQ) * (64 / PK); e += 64) {
+      const int i = iw + e / (64 / PK), j = jw + e % (64 / PK);
+      if (i < p.Qb && j < p.Kb && (!p.causal || j <= i)) out[(int64_t)i * p.Kb + j] = score_in_order(p, bg, i, j);
+    }
   }
 }
 
@@ -1084,29 +1077,7 @@ __global__ __launch_bounds__(256) void gate_scores_direct_kernel(const ScorePara
   const int64_t r = idx / p.Kb;
   const int i = (int)(r % p.Qb);
   const int64_t bg = r / p.Qb;
-  float v = -INFINITY;
-  if (!p.causal || j <= i) {
-    const float* qrow = p.qp + (bg * p.Qb + i) * (int64_t)p.Pq * p.P;
-    const float* krow = p.kp + (bg * p.Kb + j) * (int64_t)p.Pk * p.P;
-    float best = 0.f;
-    for (int a = 0; a < p.Pq; ++a)
-      for (int c = 0; c < p.Pk; ++c) {
-        const float4* x = reinterpret_cast<const float4*>(qrow + a * p.P);
-        const float4* y = reinterpret_cast<const float4*>(krow + c * p.P);
-        float acc = 0.f;
-#pragma unroll 4
-        for (int e = 0; e < p.P / 4; ++e) {
-          const float4 xv = x[e], yv = y[e];
-          acc = __builtin_fmaf(xv.x, yv.x, acc);
-          acc = __builtin_fmaf(xv.y, yv.y, acc);
-          acc = __builtin_fmaf(xv.z, yv.z, acc);
-          acc = __builtin_fmaf(xv.w, yv.w, acc);
-        }
-        best = (a == 0 && c == 0) ? acc : (acc > best ? acc : best);
-      }
-    v = best / p.div;
-  }
-  p.scores[idx] = v;
+  p.scores[idx] = !p.causal || j <= i ? score_in_order(p, bg, i, j) : -INFINITY;
 }
 
 // Causal top-k per row: radix select (4 passes of 8 bits over order keys) for
