@@ -23,6 +23,16 @@ int check_launch(const char* what);
     if (!(cond)) return ::spruce::set_error(SPRUCE_EINVAL, __VA_ARGS__); \
   } while (0)
 
+// A grid of `blocks` workgroups.  A launch of 2^32 threads or more along one
+// dimension is cut to the remainder without an error, so longer grids
+// continue along y.  Fewer than 2^32 blocks; flat_block is the position, and
+// positions past `blocks` exist.
+constexpr int64_t kGridX = 1 << 21;  // a multiple of the 8 XCDs; 1024 threads each still fit
+inline dim3 flat_grid(int64_t blocks) {
+  return blocks <= kGridX ? dim3((unsigned)blocks) : dim3((unsigned)kGridX, (unsigned)((blocks + kGridX - 1) / kGridX));
+}
+__device__ __forceinline__ uint32_t flat_block() { return blockIdx.y * (uint32_t)kGridX + blockIdx.x; }
+
 // ------------------------------------------------------------- device types
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));

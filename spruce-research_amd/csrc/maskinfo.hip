@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256) void mask_key_validity_kernel(const MaskParams
   constexpr int N = VEC ? 16 / (int)sizeof(Raw) : 1;
   struct alignas(VEC ? 16 : sizeof(Raw)) Pack { Raw v[N]; };
   const int lane = threadIdx.x & 63;
-  const int64_t g = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t g = (int64_t)flat_block() * 4 + (threadIdx.x >> 6);
   if (g >= (int64_t)p.B * p.T) return;
   const int b = (int)(g / p.T), r = (int)(g - (int64_t)b * p.T);
   const Raw* base = static_cast<const Raw*>(p.mask) + b * p.st[0];
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void mask_key_validity_kernel(const MaskParams
 // rows of K: a thread per row, one read of the lists.
 __global__ __launch_bounds__(256) void empty_rows_kernel(const int32_t* __restrict__ ids, int64_t rows, int64_t K,
                                                          int32_t* flag) {
-  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t r = (int64_t)flat_block() * 256 + threadIdx.x;
   if (r >= rows) return;
   bool listed = false;
   for (int64_t k = 0; k < K && !listed; ++k) listed = ids[r * K + k] >= 0;
@@ -149,7 +149,7 @@ using namespace spruce;
 extern "C" int spruce_empty_rows(const int32_t* ids, int64_t rows, int64_t K, int32_t* flag, void* stream) {
   SPRUCE_REQUIRE(ids && flag, "ids and flag must be non-null");
   SPRUCE_REQUIRE(rows >= 1 && K >= 1 && K < ((int64_t)1 << 31) && rows < ((int64_t)1 << 38), "invalid list shape");
-  hipLaunchKernelGGL(empty_rows_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, (hipStream_t)stream, ids,
+  hipLaunchKernelGGL(empty_rows_kernel, flat_grid((rows + 255) / 256), dim3(256), 0, (hipStream_t)stream, ids,
                      rows, K, flag);
   return check_launch("empty_rows_kernel");
 }
@@ -175,7 +175,7 @@ extern "C" int spruce_mask_key_validity(const void* mask, const int64_t ms[4], i
   p.floor = mask_dtype == 1 ? -32752.f : mask_dtype == 0 ? -0x1.fep126f : -0x1.fffffep126f;
   bool vec = (uintptr_t)mask % 16 == 0;
   for (int i = 0; i < 3; ++i) vec = vec && (ms[i] * eb) % 16 == 0;
-  const dim3 grid((unsigned)((B * T + 3) / 4));
+  const dim3 grid = flat_grid((B * T + 3) / 4);
   auto go = [&](auto m) {
     using M = decltype(m);
     if (vec)

@@ -892,7 +892,7 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
   constexpr int XL = TM * kMS / 4 / 256, YL = TN * kMS / 4 / 256;  // float4 per thread per slice
   __shared__ __attribute__((aligned(16))) float xs[TM * kMRow];
   __shared__ __attribute__((aligned(16))) float ys[TN * kMRow];
-  const int64_t id = xcd_chunk(blockIdx.x, per);
+  const int64_t id = xcd_chunk(flat_block(), per);
   if (id >= tiles) return;
   const int64_t bg = id / slab_tiles;
   const int t = (int)(id - bg * slab_tiles);
@@ -1071,7 +1071,7 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
 // tiles do not fit in LDS (e.g. 12 x 12 prototypes of 128 dims): one thread per score, operands read through
 // the cache, identical operation order.
 __global__ __launch_bounds__(256) void gate_scores_direct_kernel(const ScoreParams p, int64_t total) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t idx = (int64_t)flat_block() * 256 + threadIdx.x;
   if (idx >= total) return;
   const int j = (int)(idx % p.Kb);
   const int64_t r = idx / p.Kb;
@@ -2070,11 +2070,13 @@ extern "C" int spruce_gate_scores(const float* qp, const float* kp, int64_t BG, 
     // 128-row tiles once they give every CU two workgroups; smaller grids take 64-row tiles.
     const bool big = BG * slab(128) >= 512;
     const int64_t nti = (Qb * Pq + (big ? 127 : 63)) / (big ? 128 : 64);
-    const int64_t per_slab = slab(big ? 128 : 64), tiles = BG * per_slab, per = (tiles + 7) / 8;
+    const int64_t per_slab = slab(big ? 128 : 64), tiles = BG * per_slab;
+    int64_t per = (tiles + 7) / 8;
+    if (8 * per > kGridX) per = (per + kGridX / 8 - 1) / (kGridX / 8) * (kGridX / 8);  // whole rows of the grid
     SPRUCE_REQUIRE(8 * per < ((int64_t)1 << 31), "score matrix too large");
     auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * per)), dim3(256), 0, (hipStream_t)stream, p, (int)nti, (int)ntj,
-                         per_slab, tiles, per);
+      hipLaunchKernelGGL(kernel, flat_grid(8 * per), dim3(256), 0, (hipStream_t)stream, p, (int)nti, (int)ntj, per_slab,
+                         tiles, per);
     };
     auto pick = [&](auto pq, auto pk) {
       constexpr int A = decltype(pq)::value, C = decltype(pk)::value;
@@ -2100,7 +2102,7 @@ extern "C" int spruce_gate_scores(const float* qp, const float* kp, int64_t BG, 
     const int64_t total = BG * Qb * Kb;
     const int64_t blocks = (total + 255) / 256;
     SPRUCE_REQUIRE(blocks < ((int64_t)1 << 31), "score matrix too large");
-    hipLaunchKernelGGL(gate_scores_direct_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, p,
+    hipLaunchKernelGGL(gate_scores_direct_kernel, flat_grid(blocks), dim3(256), 0, (hipStream_t)stream, p,
                        total);
     return check_launch("gate_scores_direct_kernel");
   }

@@ -237,6 +237,18 @@ def test_mask_reduction_kernel_equals_the_tensor_operations(dtype):
                     assert torch.equal(got.cpu(), want) and padded == (not bool(want.all()))
 
 
+def test_mask_reduction_past_two_to_the_32_threads():
+    # A wavefront per mask row: 2^26 rows are 2^32 threads.  The last rows,
+    # past that, decide.
+    n = (1 << 26) + 4
+    mask = torch.ones(n, 1, 1, 1, dtype=torch.bool, device=DEV)
+    mask[[5, n - 1]] = False
+    from sparse.attention import _key_validity_and_padding
+    print(f"mask reduction over {n} rows", flush=True)
+    valid, padded, _ = _key_validity_and_padding(mask, n, 1)
+    assert padded and torch.equal(valid, mask.view(n, 1))
+
+
 def test_empty_row_check_equals_the_tensor_operations():
     # The list check beside the mask's flags, and alone: no empty row, one in
     # the first, middle or last row of a layer, rows led by padding, single

@@ -455,6 +455,21 @@ def test_matrix_scores_keep_the_sign_of_zero(Pq, Pk):
     assert negative > 100
 
 
+@pytest.mark.parametrize("Pq,Pk,P", [(8, 8, 4), (1, 3, 216)])
+def test_scores_past_two_to_the_32_threads(Pq, Pk, P):
+    # Grids of more than 2^32 threads: the matrix cores (a workgroup per 16 x
+    # 16 scores of 8 x 8 prototypes) and the kernel of one thread per score
+    # (prototypes past the tile kernel's LDS), against row ranges scored alone.
+    n = 65700
+    gen = torch.Generator(device=DEV).manual_seed(Pq)
+    qp = torch.randn(1, n, Pq, P, generator=gen, device=DEV)
+    kp = torch.randn(1, n, Pk, P, generator=gen, device=DEV)
+    print(f"scores {n} x {n}, {Pq} x {Pk} prototypes", flush=True)
+    got = gate_scores(qp, kp, causal=False)
+    for i in range(0, n, 8192):
+        assert torch.equal(got[:, i:i + 8192], gate_scores(qp[:, i:i + 8192].contiguous(), kp, causal=False))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("L,S,nodes,Pk,D,P", [
     (1, 1, [1], 1, 4, 4), (3, 2, [37, 19, 1], 8, 36, 64), (2, 1, [70], 4, 128, 132), (2, 3, [1500, 750, 5], 8, 32, 260)])
