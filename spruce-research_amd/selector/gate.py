@@ -42,7 +42,10 @@ class FlatGate(nn.Module):
         if 1 <= L <= W.shape[0] and feat.shape[-1] == d and d % 4 == 0 and p % 4 == 0 and feat.numel() and \
                 feat.dtype in (torch.bfloat16, torch.float16, torch.float32):
             rows = feat.reshape(L, 1, -1, 1, d).contiguous()
-            if rows.data_ptr() % 16 == 0:   # every layer in one launch
+            # The limits of project_layers; float32 calls past them take the general kernels.
+            past = feat.dtype == torch.float32 and (
+                max(d, p) > 4096 or rows.shape[2] >= 1 << 30 or W.data_ptr() % 16 != 0)
+            if rows.data_ptr() % 16 == 0 and not past:   # every layer in one launch
                 return project_layers([rows], W[:L]).reshape(feat.shape[:-1] + (p,))
         if L == 1:
             return project(feat[0].float(), W[0].float()).unsqueeze(0)

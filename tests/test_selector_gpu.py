@@ -497,6 +497,23 @@ def test_projection_of_layers_equals_each_layer(dtype, L, S, nodes, Pk, D, P):
         assert torch.equal(gate.project_queries(odd), want)   # not 16-byte aligned: the general kernels
 
 
+@pytest.mark.parametrize("L", [1, 2])
+@pytest.mark.parametrize("d,p,shift", [(4100, 8, 0), (8, 4100, 0), (4096, 8, 0), (8, 4096, 0), (16, 12, 1)])
+def test_float32_gate_projections_past_the_one_launch_limits(L, d, p, shift):
+    # Dims past 4096 (and at it), and a weight that is a view four bytes into
+    # a flat buffer: float32 features take the general kernels, one per layer.
+    gen = torch.Generator().manual_seed(d + p + L)
+    feat = torch.randn(L, 2, 5, 3, d, generator=gen).to(DEV)
+    gate = FlatGate(L, d, proj_dim=p).to(DEV).requires_grad_(False)
+    flat = torch.randn(L * d * p + shift, generator=gen).to(DEV)
+    gate.Wq.data = flat[shift:].view(L, d, p)
+    assert gate.Wq.data_ptr() % 16 == 4 * shift
+    print(f"gate projection L={L} d={d} p={p} shift={shift}", flush=True)
+    got = gate.project_queries(feat)
+    want = np.stack([osel.project(_np(feat[l]), _np(gate.Wq[l])) for l in range(L)])
+    np.testing.assert_array_equal(_np(got), want)
+
+
 @pytest.mark.parametrize("Kb", [1, 63, 64, 65, 255, 256, 257, 512, 513, 1024])
 def test_topk_slots_per_lane(Kb):
     # Rows held in 4, 8 or 16 slots a lane: the widths where the slot count
