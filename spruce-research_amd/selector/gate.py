@@ -45,7 +45,8 @@ class FlatGate(nn.Module):
             # The limits of project_layers; float32 calls past them take the general kernels.
             past = feat.dtype == torch.float32 and (
                 max(d, p) > 4096 or rows.shape[2] >= 1 << 30 or W.data_ptr() % 16 != 0)
-            if rows.data_ptr() % 16 == 0 and not past:   # every layer in one launch
+            # The kernel reads four values at a time: 8 bytes of 16-bit features.
+            if rows.data_ptr() % (4 * rows.element_size()) == 0 and not past:   # every layer in one launch
                 return project_layers([rows], W[:L]).reshape(feat.shape[:-1] + (p,))
         if L == 1:
             return project(feat[0].float(), W[0].float()).unsqueeze(0)

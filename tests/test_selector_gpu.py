@@ -514,6 +514,27 @@ def test_float32_gate_projections_past_the_one_launch_limits(L, d, p, shift):
     np.testing.assert_array_equal(_np(got), want)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("L", [1, 3])
+def test_features_aligned_to_8_bytes_are_read_directly(monkeypatch, dtype, L):
+    # 16-bit features 8 bytes past a 16-byte boundary, 70 rows a layer: one
+    # launch over them, no float32 copy and no projection per layer.
+    import selector.gate as gate_module
+    gen = torch.Generator().manual_seed(L)
+    d, p = 36, 68
+    flat = torch.randn(4 + L * 70 * d, generator=gen).to(dtype).to(DEV)
+    feat = flat[4:].view(L, 2, 5, 7, d)
+    assert feat.data_ptr() % 16 == 8
+    gate = FlatGate(L, d, proj_dim=p).to(DEV).requires_grad_(False)
+    want = np.stack([osel.project(_np(feat[l].float()), _np(gate.Wq[l])) for l in range(L)])
+
+    def per_layer(*args):
+        raise AssertionError("a projection per layer of a float32 copy")
+    monkeypatch.setattr(gate_module, "project", per_layer)
+    print(f"features at 8 bytes, {dtype} L={L}", flush=True)
+    np.testing.assert_array_equal(_np(gate.project_queries(feat)), want)
+
+
 @pytest.mark.parametrize("Kb", [1, 63, 64, 65, 255, 256, 257, 512, 513, 1024])
 def test_topk_slots_per_lane(Kb):
     # Rows held in 4, 8 or 16 slots a lane: the widths where the slot count
