@@ -605,9 +605,13 @@ __device__ __forceinline__ f32x4_t widen4(const ProjRowsSeg<TIn>&, V w) {
 // stores.  D = P = 128, bf16 rows: 28 layers of 4096 rows, both sides, 56
 // launches of 20 us (8 x 4 outputs a thread) and two stacking copies, 1164 us
 // -> two launches, 121 us; 131,040 node rows interleaved 85 -> 62 us.
-// From 16384 rows the 128-column tiles fill the CUs; fewer float32 rows of one
-// layer take the 64-column tiles above.
-constexpr int kMfmaProjectRows = 16384;
+// One layer of float32 rows takes the 64 x 64 tiles above while fewer than 256
+// of them leave CUs free (the pair of projections: its 32-row tiles below
+// 16384 rows).  P = 128: 64 rows 8.8 us there and 9.9 here, 4096 rows 10.2
+// and 10.5, 8192 rows (256 tiles) 10.8 and 9.7, 12288 rows 12.8 and 10.1;
+// P = 64: 64 rows 5.7 and 6.6, 8192 rows 6.6 and 7.3, 16383 rows (256 tiles)
+// 7.0 and 6.8.
+constexpr int kMfmaProjectRows = 8192, kMfmaProjectTiles = 256, kMfmaPairRows = 16384;
 template <int RA, typename Rows, bool IL>
 __global__ __launch_bounds__(256, RA == 2 ? 3 : 4) void project_mfma_kernel(const Rows src, const float* __restrict__ w,
                                                                             int64_t rows, int D, int P,
@@ -1951,7 +1955,7 @@ extern "C" int spruce_gate_project(const float* x, const float* w, int64_t N, in
   SPRUCE_REQUIRE(N >= 1 && D >= 1 && P >= 1 && N * P < ((int64_t)1 << 40), "invalid projection shape");
   const bool vec = D % 4 == 0 && P % 4 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0 &&
                    ((uintptr_t)out % 16) == 0;
-  if (vec && N >= kMfmaProjectRows) {
+  if (vec && N >= kMfmaProjectRows && ((N + 63) / 64) * ((P + 63) / 64) >= kMfmaProjectTiles) {
     SPRUCE_REQUIRE(P < ((int64_t)1 << 20) && D < ((int64_t)1 << 20), "projection too large");
     return launch_project_mfma(ProjRowsF32{x}, w, 1, N, (int)D, (int)P, out, false, 0, (hipStream_t)stream);
   }
@@ -2029,7 +2033,7 @@ extern "C" int spruce_gate_project2(const float* xa, const float* wa, int64_t Na
   auto aligned = [](const void* q) { return ((uintptr_t)q % 16) == 0; };
   const bool vec = D % 4 == 0 && P % 4 == 0 && aligned(xa) && aligned(wa) && aligned(outa) && aligned(xb) &&
                    aligned(wb) && aligned(outb);
-  if (!vec || Na >= kMfmaProjectRows || Nb >= kMfmaProjectRows) {
+  if (!vec || Na >= kMfmaPairRows || Nb >= kMfmaPairRows) {
     const int rc = spruce_gate_project(xa, wa, Na, D, P, outa, stream);
     return rc != 0 ? rc : spruce_gate_project(xb, wb, Nb, D, P, outb, stream);
   }

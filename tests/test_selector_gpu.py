@@ -514,6 +514,22 @@ def test_float32_gate_projections_past_the_one_launch_limits(L, d, p, shift):
     np.testing.assert_array_equal(_np(got), want)
 
 
+@pytest.mark.parametrize("N,P", [(8191, 128), (8192, 128), (8192, 64), (16320, 64), (16321, 64), (8192, 68), (8191, 4100)])
+def test_float32_projection_of_one_layer_around_the_tile_line(monkeypatch, N, P):
+    # 64 x 64 tiles up to 255 of them or below 8192 rows, matrix cores from
+    # there: the gate's float32 call of one layer takes this route, the values
+    # those of small row ranges.
+    import selector.gate as gate_module
+    gen = torch.Generator().manual_seed(N + P)
+    x = torch.randn(1, 1, N, 1, 36, generator=gen).to(DEV)
+    gate = FlatGate(1, 36, proj_dim=P).to(DEV).requires_grad_(False)
+    want = torch.cat([project(c, gate.Wq[0]) for c in x.view(N, 36).split(1000)])
+    monkeypatch.setattr(gate_module, "project_layers", None)
+    print(f"float32 gate projection N={N} P={P}", flush=True)
+    assert torch.equal(gate.project_queries(x).view(N, P), want)
+    np.testing.assert_array_equal(_np(want[:70]), osel.project(_np(x.view(N, 36)[:70]), _np(gate.Wq[0])))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("L", [1, 3])
 def test_features_aligned_to_8_bytes_are_read_directly(monkeypatch, dtype, L):
