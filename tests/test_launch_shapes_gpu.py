@@ -198,3 +198,38 @@ def test_helper_wave_launches_agree_with_the_eight_wave_forms(Hq, Hkv, tokens, v
         assert torch.equal(alone, together[:1]), name
     assert torch.equal(pairs["index"][0], pairs["mask"][0].transpose(1, 2))
     assert torch.equal(pairs["index"][0], pairs["csr"][0])
+
+
+@pytest.mark.parametrize("dtype,head_dim", [(torch.bfloat16, 128), (torch.float16, 64), (torch.float32, 128)])
+@pytest.mark.parametrize("Hq,Hkv,tokens,density", [
+    (8, 2, 4096, 0.1),     # 4-tile parts of two heads, with helper waves
+    (16, 2, 2000, 0.3),    # four parts, ragged
+    (12, 2, 333, 0.3),     # 2-tile parts
+    (4, 2, 1000, 0.2),     # rows of four tiles
+])
+def test_masks_of_each_query_head_in_split_launches(Hq, Hkv, tokens, density, dtype, head_dim):
+    # Every query head has a mask of its own: a part walks the blocks that any
+    # of its heads lists and drops the others' per head.  Batch element 0 must
+    # equal the one of a batch that fills the GPU, and each head what it gets
+    # when every head of its group has its mask.
+    print(f"head masks: Hq={Hq} Hkv={Hkv} T={tokens} D={head_dim} {dtype}", flush=True)
+    qb = (tokens + 63) // 64
+    B = max(2, min(12, -(-512 // (Hkv * qb))))
+    gen = torch.Generator().manual_seed(tokens + Hq)
+    q, k, v = [torch.randn(B, tokens, H, head_dim, generator=gen).to(dtype).to(DEV).transpose(1, 2)
+               for H in (Hq, Hkv, Hkv)]
+    mask = torch.rand(B, Hq, qb, qb, generator=gen) < density
+    mask |= torch.eye(qb, dtype=torch.bool)
+    mask &= torch.ones(qb, qb).tril().bool()
+    mask[:, Hq // 2, qb // 2] = False        # a head's row with no block
+    mask = mask.to(DEV)
+    scale = head_dim ** -0.5
+    alone = block_sparse_prefill(q[:1], k[:1], v[:1], mask[:1], scale)
+    together = block_sparse_prefill(q, k, v, mask, scale)
+    assert torch.isfinite(alone.float()).all()
+    assert torch.equal(alone, together[:1])
+    G = Hq // Hkv
+    for i in range(G):
+        group = mask[:1, i::G].repeat_interleave(G, dim=1)
+        same = block_sparse_prefill(q[:1], k[:1], v[:1], group, scale)
+        assert torch.equal(alone[:, i::G], same[:, i::G])
