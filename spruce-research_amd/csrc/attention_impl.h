@@ -101,7 +101,7 @@ struct AttnParams {
   const float* slog;
   float sbias;  // log counts -> raw score units: log2(e) / cs
   int tpp;  // tiles per part: waves 0..tpp-1 of a workgroup own a tile
-  int help;  // small grid: as many helper waves as tile waves (4- and 2-tile parts)
+  int help;  // as many helper waves as tile waves (4- and 2-tile parts)
   // feature capture (dense causal form): group-averaged queries
   // [B, Hkv, T, D] and key prototypes [B, Hkv, Qb, P, D], model dtype,
   // contiguous; each part covers tpp / G whole 32-row halves of the block.
@@ -548,9 +548,9 @@ __device__ __forceinline__ void lds_barrier() {
 
 // HELP: the second half of the workgroup's waves own no tile and stage every
 // K/V block through their registers, a block ahead of the one the tile waves
-// compute.  In a small grid a tile wave has its SIMD to itself, so what bounds
-// it is its own chain per block; the wait for the staged loads, the rounding
-// of float32 blocks and the LDS stores leave that chain.
+// compute.  Where few tile waves share a SIMD, what bounds one is its own
+// chain per block; the wait for the staged loads, the rounding of float32
+// blocks and the LDS stores leave that chain.
 template <int D, int WAVES, typename TIn, bool F16, int MODE, bool SUMM = false, bool CAP = false, bool PROD = false,
           bool KVAL = false, bool AMASK = false, bool HELP = false>
 __global__ __launch_bounds__(WAVES * 64, HELP && !AMASK ? 2 : 1) void sparse_prefill_kernel(const AttnParams p) {
@@ -1422,14 +1422,27 @@ inline LaunchShape choose_shape(int variant, int G) {
 // idle CU.  Every shape computes the same attention.
 constexpr int64_t kComputeUnits = 256;  // MI355X
 //
-// Helper waves (the HELP form) double a 4- or 2-tile workgroup; they are taken
-// while the grid still leaves every SIMD at most two waves (one workgroup of
-// eight waves or two of four on a CU; `one_per_cu`: a form whose LDS lets only
-// one workgroup on a CU).  Measured (index form, before ->
-// after): 8/2 heads, T = 4096, 27 blocks a row, float32 58.0 -> 41.1, bf16 47.4
-// -> 34.5 us; 12/2, T = 333, 6 blocks 13.6 -> 10.5; 28/4, T = 1000, 10 blocks
-// 21.8 -> 19.6.
-inline void split_small_grid(AttnParams& p, LaunchShape& s, int variant, bool one_per_cu = false) {
+// Helper waves (the HELP form) double a 4- or 2-tile workgroup of the list
+// forms without summaries.  They pay where they take no resident workgroup's
+// place:
+//  * four tiles, D = 128: a plain workgroup's waves hold 288 and more
+//    registers, one a SIMD, so one workgroup runs on a CU either way and the
+//    helpers take the other half of its registers.  At any size: padded lists
+//    of 12 blocks a row, plain -> helpers, 8/2 heads, T = 4085 (256 workgroups),
+//    float32 33.7 -> 26.4, bf16 26.1 -> 20.1 us; T = 5109 (320) 58.5 -> 43.1 and
+//    47.3 -> 35.2; 24 blocks a row, 4/2 heads, T = 64K (2048) 434 -> 352 and 334
+//    -> 266; 16/8, T = 64K (8192) 1778 -> 1452 and 1330 -> 1059.  Block masks,
+//    CSR lists and key padding 1.2 - 1.5x, the general mask 1.04 - 1.11x.
+//  * four tiles, D = 64: two plain workgroups run on a CU, and two with
+//    helpers only where those need at most 128 registers (not with block
+//    masks or key padding).  Up to one workgroup a CU (1.17 - 1.40x, the
+//    general mask 1.03x); 16/2 heads, T = 2997 (376 workgroups), key padding:
+//    32.4 -> 37.7 us.
+//  * two tiles: up to two workgroups a CU, which is what runs there either
+//    way (12/2 heads, T = 333, 6 blocks 13.6 -> 10.5; 28/4, T = 1013, 12 blocks
+//    26.7 -> 22.8, float32 33.0 -> 24.2 us).  Past that float32 rows of 40
+//    blocks lose (8/8 heads, T = 38K: 887 -> 1133 us).
+inline void split_small_grid(AttnParams& p, LaunchShape& s, int variant, int64_t D) {
   if (variant == SPRUCE_VARIANT_SINGLE_HEAD_QTILE) return;
   const int64_t rows = (int64_t)p.B * p.Hkv * p.Qb;
   const int tiles = 2 * p.G;
@@ -1441,8 +1454,9 @@ inline void split_small_grid(AttnParams& p, LaunchShape& s, int variant, bool on
   }
   p.parts = s.parts;
   p.tpp = s.tpp;
-  const int64_t per_cu = one_per_cu || s.waves == 4 ? 1 : 2;
-  p.help = s.waves < 8 && s.tpp == s.waves && rows * s.parts <= kComputeUnits * per_cu;
+  const int64_t groups = rows * s.parts;
+  p.help = s.tpp == s.waves && (s.waves == 4 ? D == 128 || groups <= kComputeUnits
+                                             : s.waves == 2 && groups <= 2 * kComputeUnits);
 }
 
 template <int D, int WAVES, typename TIn, bool F16, int MODE, bool SUMM, bool CAP = false, bool PROD = false,
@@ -1458,14 +1472,19 @@ int launch_attention_t(const AttnParams& p, hipStream_t stream) {
 
 template <int MODE, bool SUMM, int D, typename TIn, bool F16, bool KVAL, bool AMASK = false>
 int launch_attention_w(const AttnParams& p, int waves, hipStream_t stream) {
-  if constexpr (!SUMM && MODE != kModeCausal)
+  constexpr bool kHelpers = !SUMM && MODE != kModeCausal;
+  if constexpr (kHelpers)
     if (p.help) {
       if (waves == 2) return launch_attention_t<D, 4, TIn, F16, MODE, false, false, false, KVAL, AMASK, true>(p, stream);
       if (waves == 4) return launch_attention_t<D, 8, TIn, F16, MODE, false, false, false, KVAL, AMASK, true>(p, stream);
     }
   switch (waves) {
     case 2: return launch_attention_t<D, 2, TIn, F16, MODE, SUMM, false, false, KVAL, AMASK>(p, stream);
-    case 4: return launch_attention_t<D, 4, TIn, F16, MODE, SUMM, false, false, KVAL, AMASK>(p, stream);
+    case 4:
+      if constexpr (kHelpers && D == 128)
+        return set_error(SPRUCE_EINVAL, "four tiles of head_dim 128 take helper waves");  // not reached
+      else
+        return launch_attention_t<D, 4, TIn, F16, MODE, SUMM, false, false, KVAL, AMASK>(p, stream);
     case 8:
       // A spare wave becomes the K/V producer (16-bit inputs, key blocks only).
       if constexpr (kUseProducer && TIn::bytes == 2)

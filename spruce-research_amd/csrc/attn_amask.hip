@@ -18,7 +18,7 @@ extern "C" int spruce_sparse_prefill_index_amask(
   int rc = prepare_attention(p, q, qs, k, ks, v, vs, B, Hq, Hkv, T, D, scale, dtype, variant, out, os,
                              shape);
   if (rc) return rc;
-  split_small_grid(p, shape, variant, true);  // the mask rows take LDS of their own
+  split_small_grid(p, shape, variant, D);
   SPRUCE_REQUIRE(idx != nullptr && is != nullptr, "indices must be a non-null device pointer");
   SPRUCE_REQUIRE(K >= 0 && K < (int64_t)1 << 30, "invalid index row width K=%lld", (long long)K);
   SPRUCE_REQUIRE(amask != nullptr && ams != nullptr, "the attention mask must be a non-null device pointer");

@@ -14,7 +14,7 @@ extern "C" int spruce_sparse_prefill_csr(
   int rc = prepare_attention(p, q, qs, k, ks, v, vs, B, Hq, Hkv, T, D, scale, dtype, variant, out, os,
                              shape);
   if (rc) return rc;
-  split_small_grid(p, shape, variant);
+  split_small_grid(p, shape, variant, D);
   SPRUCE_REQUIRE(nnz >= 0 && nnz < ((int64_t)1 << 31), "invalid nnz %lld", (long long)nnz);
   // With no entries (every row empty) indices is never read and may be null.
   SPRUCE_REQUIRE(indptr != nullptr && (indices != nullptr || nnz == 0), "indptr and indices must be non-null");

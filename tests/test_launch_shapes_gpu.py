@@ -141,21 +141,24 @@ def test_split_and_unsplit_launches_agree(entry, Hq, Hkv, B, dtype):
 
 @pytest.mark.parametrize("dtype,head_dim", [(torch.bfloat16, 128), (torch.float16, 64), (torch.float32, 128)])
 @pytest.mark.parametrize("Hq,Hkv,tokens,variant", [
-    (8, 2, 4096, "single_head"),        # 128 rows: 4-tile parts with helper waves fill 256 CUs exactly
-    (8, 2, 4100, "single_head"),        # one row more: no helper waves
+    (8, 2, 4096, "single_head"),        # 128 rows in 4-tile parts with helper waves: one per CU
+    (8, 2, 4100, "single_head"),        # a block more: helper waves at head_dim 128 only
+    (16, 4, 2048, "single_head"),       # the same two with the general mask
+    (16, 4, 2060, "single_head"),
+    (4, 2, 5000, "single_head"),        # rows of four tiles, fewer than CUs: 2-tile parts with helper waves
     (12, 2, 333, "single_head"),        # 2-tile parts with helper waves, ragged
     (28, 4, 1170, "single_head"),       # 2-tile parts, 532 workgroups: no helper waves
     (2, 1, 8, "single_head"),           # one row of one block
     (8, 2, 600, "single_head_qtile"),   # keeps its own shape
 ])
 def test_helper_wave_launches_agree_with_the_eight_wave_forms(Hq, Hkv, tokens, variant, dtype, head_dim):
-    # Small grids take helper waves (or just miss them); batch element 0 must
-    # equal the one of a batch that fills the GPU, for every list form, with
-    # empty rows, rows of one block and rows of several.
+    # Either side of the sizes at which helper waves are taken; batch element
+    # 0 must equal the one of a batch large enough for another form, for every
+    # list form, with empty rows, rows of one block and rows of several.
     print(f"helper waves: Hq={Hq} Hkv={Hkv} T={tokens} D={head_dim} {dtype} {variant}", flush=True)
     qb = (tokens + 63) // 64
     B = max(2, -(-512 // (Hkv * qb)))
-    B = min(B, 12)
+    B = min(B, 12 if tokens > 64 else 600)
     gen = torch.Generator().manual_seed(tokens + Hq)
     q, k, v = [torch.randn(B, tokens, H, head_dim, generator=gen).to(dtype).to(DEV).transpose(1, 2)
                for H in (Hq, Hkv, Hkv)]
@@ -175,7 +178,7 @@ def test_helper_wave_launches_agree_with_the_eight_wave_forms(Hq, Hkv, tokens, v
     ind = keep.nonzero()[:, 3].int()
     n1 = Hkv * qb
     valid = (torch.arange(tokens)[None] >= torch.randint(0, tokens // 2 + 1, (B, 1), generator=gen)).to(DEV)
-    bias = torch.randn(B, 1, tokens, tokens, generator=gen).to(torch.bfloat16).to(DEV) if tokens <= 1200 else None
+    bias = torch.randn(B, 1, tokens, tokens, generator=gen).to(torch.bfloat16).to(DEV) if tokens <= 2100 else None
     kw = dict(kernel_variant=variant)
     pairs = {
         "index": (direct_index_sparse_prefill(q[:1], k[:1], v[:1], idx[:1], scale, **kw),
