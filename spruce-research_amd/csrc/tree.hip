@@ -435,18 +435,17 @@ __device__ __forceinline__ float maxsim_one(const float* qrow, const float* krow
 // the results are identical.  The key vectors stream in pieces of CW float4
 // (loads back to back): lanes read different vectors, and taking a line in a
 // few pieces close together keeps it in L1 between them, where one float4
-// per step was refetched from L2 for every 16 bytes (measured 1.85 -> 1.0-1.1
-// ms at the cfg5 grid).  Two register sets take the pieces in turn, the next
-// piece loading while the other is used, so no piece is copied between
-// registers (the loads are unconditional: the last one re-reads piece 0,
-// in bounds and unused).  Requires pd % (8 * CW) == 0; PD > 0 fixes pd at
-// compile time, so the query reads take immediate LDS offsets, and GS > 0
-// the key group stride (4: rows layout; 4 * Pk: interleaved, where the Pk
-// prototypes of a node that neighbouring lanes hold share each 16 * Pk-byte
-// group, so a load touches one line per node instead of one per lane).
-template <int NP, int CW, int GS>
-__device__ __forceinline__ void load_piece(const float* const (&kv)[NP], int e0, int gs_rt, float4 (&k)[NP][CW]) {
-  const int gs = GS > 0 ? GS : gs_rt;
+// per step was refetched from L2 for every 16 bytes (1.85 -> 1.0-1.1 ms with
+// 8 x 8 prototypes of 128 dims at 2048 leaves, which the matrix cores score
+// now).  Two register sets take the pieces in turn, the next piece loading
+// while the other is used, so no piece is copied between registers (the loads
+// are unconditional: the last one re-reads piece 0, in bounds and unused).
+// Requires pd % (8 * CW) == 0.  gs is the key group stride (4: rows layout;
+// 4 * Pk: interleaved, where the Pk prototypes of a node that neighbouring
+// lanes hold share each 16 * Pk-byte group, so a load touches one line per
+// node instead of one per lane).
+template <int NP, int CW>
+__device__ __forceinline__ void load_piece(const float* const (&kv)[NP], int e0, int gs, float4 (&k)[NP][CW]) {
 #pragma unroll
   for (int n = 0; n < NP; ++n)
 #pragma unroll
@@ -454,10 +453,9 @@ __device__ __forceinline__ void load_piece(const float* const (&kv)[NP], int e0,
       k[n][j] = *reinterpret_cast<const float4*>(kv[n] + (int64_t)(e0 / 4 + j) * gs);
 }
 
-template <int PQ, int NP, int CW, int PD>
-__device__ __forceinline__ void fma_piece(const float* qrow, int pd_rt, int e0, const float4 (&k)[NP][CW],
+template <int PQ, int NP, int CW>
+__device__ __forceinline__ void fma_piece(const float* qrow, int pd, int e0, const float4 (&k)[NP][CW],
                                           float (&acc)[NP][PQ]) {
-  const int pd = PD > 0 ? PD : pd_rt;
 #pragma unroll
   for (int j = 0; j < CW; ++j) {
     const int e = e0 + 4 * j;
@@ -477,10 +475,9 @@ __device__ __forceinline__ void fma_piece(const float* qrow, int pd_rt, int e0, 
   }
 }
 
-template <int PQ, int NP, int CW, int PD, int GS>
-__device__ __forceinline__ void maxsim_multi(const float* qrow, const float* const (&kv)[NP], int pd_rt, int gs,
+template <int PQ, int NP, int CW>
+__device__ __forceinline__ void maxsim_multi(const float* qrow, const float* const (&kv)[NP], int pd, int gs,
                                              float (&res)[NP]) {
-  const int pd = PD > 0 ? PD : pd_rt;
   float acc[NP][PQ];
 #pragma unroll
   for (int n = 0; n < NP; ++n)
@@ -488,12 +485,12 @@ __device__ __forceinline__ void maxsim_multi(const float* qrow, const float* con
     for (int a = 0; a < PQ; ++a) acc[n][a] = 0.f;
   constexpr int kStep = 4 * CW;
   float4 ka[NP][CW], kb[NP][CW];
-  load_piece<NP, CW, GS>(kv, 0, gs, ka);
+  load_piece<NP, CW>(kv, 0, gs, ka);
   for (int e0 = 0; e0 < pd; e0 += 2 * kStep) {
-    load_piece<NP, CW, GS>(kv, e0 + kStep, gs, kb);
-    fma_piece<PQ, NP, CW, PD>(qrow, pd, e0, ka, acc);
-    load_piece<NP, CW, GS>(kv, e0 + 2 * kStep < pd ? e0 + 2 * kStep : 0, gs, ka);
-    fma_piece<PQ, NP, CW, PD>(qrow, pd, e0 + kStep, kb, acc);
+    load_piece<NP, CW>(kv, e0 + kStep, gs, kb);
+    fma_piece<PQ, NP, CW>(qrow, pd, e0, ka, acc);
+    load_piece<NP, CW>(kv, e0 + 2 * kStep < pd ? e0 + 2 * kStep : 0, gs, ka);
+    fma_piece<PQ, NP, CW>(qrow, pd, e0 + kStep, kb, acc);
   }
 #pragma unroll
   for (int n = 0; n < NP; ++n) {
@@ -615,9 +612,10 @@ __device__ __forceinline__ float max_over_prototypes(float x) {
   return x != x ? x : m;
 }
 
-// Two pairs per lane in 64-byte pieces.  Measured at the cfg5 grid against
-// 1.0-1.06 ms: four pairs in 64-byte pieces 1.68 ms (289 registers), four in
-// 32-byte pieces 1.10 ms, four or eight in 16-byte pieces 1.77-2.03 ms.
+// Two pairs per lane in 64-byte pieces.  Of maxsim_multi with 8 x 8 prototypes
+// of 128 dims at 2048 leaves (1.0-1.06 ms): four pairs in 64-byte pieces 1.68
+// ms (289 registers), four in 32-byte pieces 1.10 ms, four or eight in 16-byte
+// pieces 1.77-2.03 ms.
 constexpr int kTravNP = 2, kTravCW = 4;
 
 struct TraverseParams {
@@ -674,7 +672,8 @@ __device__ __forceinline__ void score_pairs(const ScoreParams2& sc, const float*
 // At 2048 leaves and beam 16 that leaves 224 of 254 scored candidates a row.
 template <int PQ, int PD = 0, int GS = 0>
 __global__ __launch_bounds__(64, PD > 0 ? 4 : 1) void tree_traverse_kernel(const TraverseParams p) {
-  constexpr bool kMfma = PD > 0 && PQ % 4 == 0 && PQ > 0;
+  constexpr bool kMfma = PD > 0;
+  static_assert(!kMfma || PQ == 4 || PQ == 8, "the matrix cores take 4 or 8 query prototypes");
   constexpr int PK = kMfma && GS > 4 ? GS / 4 : 0;  // key prototypes, where the group stride tells them
   extern __shared__ float sh[];
   const ScoreParams2& sc = p.sc;
@@ -744,12 +743,12 @@ __global__ __launch_bounds__(64, PD > 0 ? 4 : 1) void tree_traverse_kernel(const
       constexpr int Q = PQ == 0 ? 1 : PQ;
       if (one)
         score_pairs<1, 0>(sc, kl, cand, nv, lane, pm, [&](const float* const (&kv)[1], float (&m)[1]) {
-          maxsim_multi<Q, 1, kTravCW, PD, GS>(qrow, kv, sc.pd, sc.gs, m);
+          maxsim_multi<Q, 1, kTravCW>(qrow, kv, sc.pd, sc.gs, m);
         });
       else
         score_pairs<kTravNP, 0>(sc, kl, cand, nv, lane, pm,
                                 [&](const float* const (&kv)[kTravNP], float (&m)[kTravNP]) {
-                                  maxsim_multi<Q, kTravNP, kTravCW, PD, GS>(qrow, kv, sc.pd, sc.gs, m);
+                                  maxsim_multi<Q, kTravNP, kTravCW>(qrow, kv, sc.pd, sc.gs, m);
                                 });
     } else {
       for (int pr = lane; pr < nv * sc.Pk; pr += 64) {
