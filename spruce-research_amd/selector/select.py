@@ -146,6 +146,9 @@ def project_levels(levels, W, interleaved=False):
     the tree traversal reads fastest."""
     if not levels:
         raise ValueError("levels must not be empty")
+    for t in levels:
+        if t.dim() != 4:
+            raise ValueError("levels must be [S, n, P, D] with one S, P, D and dtype")
     if W.dim() != 2 or W.shape[0] != levels[0].shape[-1]:
         raise ValueError(f"shape mismatch: levels [..., {levels[0].shape[-1]}] @ W {tuple(W.shape)}")
     return project_layers([t.unsqueeze(0) for t in levels], W.unsqueeze(0), interleaved=interleaved)[0]
@@ -160,11 +163,10 @@ def project_layers(levels, W, interleaved=False):
         raise ValueError("levels must not be empty")
     for t in levels:
         _cuda(t, "levels")
+        if t.dim() != 5 or t.shape[:2] != levels[0].shape[:2] or t.shape[3:] != levels[0].shape[3:] or \
+                t.dtype != levels[0].dtype:
+            raise ValueError("levels must be [L, S, n, P, D] with one L, S, P, D and dtype")
     L, S, _, P, D = levels[0].shape
-    dtype = levels[0].dtype
-    for t in levels:
-        if t.dim() != 5 or t.shape[:2] != (L, S) or t.shape[3:] != (P, D) or t.dtype != dtype:
-            raise ValueError("levels must be [S, n, P, D] with one S, P, D and dtype")
     if W.dim() != 3 or W.shape[:2] != (L, D):
         raise ValueError(f"shape mismatch: levels [..., {D}] of {L} layers @ W {tuple(W.shape)}")
     W = W.to(device=levels[0].device, dtype=torch.float32).contiguous()

@@ -497,6 +497,19 @@ def test_projection_of_layers_equals_each_layer(dtype, L, S, nodes, Pk, D, P):
         assert torch.equal(gate.project_queries(odd), want)   # not 16-byte aligned: the general kernels
 
 
+def test_projection_of_levels_names_the_shape_it_takes():
+    from selector.select import project_layers, project_levels
+    t = torch.zeros(2, 3, 4, 8, device=DEV)
+    W = torch.zeros(8, 8, device=DEV)
+    for bad in ([t[0]], [t, t[0]], [t[None]]):
+        with pytest.raises(ValueError, match=r"levels must be \[S, n, P, D\]"):
+            project_levels(bad, W)
+    for bad in ([t], [t[None], t], [t[None], t[None, :1]], [t[None], t[None].half()], [t[None], t[None, :, :, :2]]):
+        with pytest.raises(ValueError, match=r"levels must be \[L, S, n, P, D\]"):
+            project_layers(bad, W[None])
+    assert project_layers([t[None], t[None, :, :2]], W[None]).shape == (1, 2, 5, 4, 8)
+
+
 @pytest.mark.parametrize("L", [1, 2])
 @pytest.mark.parametrize("d,p,shift", [(4100, 8, 0), (8, 4100, 0), (4096, 8, 0), (8, 4096, 0), (16, 12, 1)])
 def test_float32_gate_projections_past_the_one_launch_limits(L, d, p, shift):
