@@ -872,8 +872,8 @@ __device__ __forceinline__ float dpp_max(float x) {
 }
 
 // The scores above for 1, 2, 4 or 8 prototypes a side, as one matrix product
-// of prototype rows: a workgroup of 2 x 2 waves covers 64 RA query rows x 128
-// key rows, each wave 32 RA x 64, and reduces its accumulators to one maximum
+// of prototype rows: a workgroup of 2 x 2 waves covers 64 RA query rows x 64 RA
+// key rows, each wave 32 RA x 32 RA, and reduces its accumulators to one maximum
 // per (query block, key block): the PQ rows of a query block are registers of
 // one lane (and its other half for PQ = 8), the PK columns neighbouring lanes.
 // fmaxf drops NaN as "replace when strictly larger" does, except for the
@@ -887,26 +887,59 @@ __device__ __forceinline__ float dpp_max(float x) {
 // 28 x 2 slabs of 256 x 256 blocks, causal: 10.17 ms with one thread per
 // score (every pair a dependent chain whose operands come through the cache)
 // -> 0.319 ms.  One query and two key prototypes, 4 slabs of 1024 blocks:
-// 31.9 (VALU, 2 x 4 x 2 outputs a thread) -> 23.8 us.
+// 31.9 (VALU, 2 x 4 x 2 outputs a thread) -> 23.8 us with 64 x 128 tiles in
+// small grids; launch to launch in a captured graph 21.5 -> 18.9 us with the
+// 64 x 64 ones, of which a wave's outputs and code are half, most of a short
+// kernel (one prototype of 32 dims, 4 slabs of 64 blocks: 5.1 -> 3.9 us).
+//
+// causal == 1 with Qb == Kb: what lies right of a row's tiles is filled by
+// workgroups of its own past the tiles, 16 rows each (filled by the row's last
+// tile, the first row tiles ran longest: one prototype of 32 dims, 512 blocks
+// 8.9 -> 4.4 us with the smaller tiles; one and two of 128 dims, 4 x 512 blocks
+// 13.7 -> 9.5 us).
+constexpr int kFillRows = 16;
 template <int PQ, int PK, int RA>
 __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate_scores_mfma_kernel(const ScoreParams p, int nti, int ntj,
                                                                                 int64_t slab_tiles, int64_t tiles,
                                                                                 int64_t per) {
-  constexpr int TM = 64 * RA, TN = 128, TI = TM / PQ, TJ = TN / PK;
+  constexpr int TM = 64 * RA, TN = 64 * RA, TI = TM / PQ, TJ = TN / PK;
   constexpr int XL = TM * kMS / 4 / 256, YL = TN * kMS / 4 / 256;  // float4 per thread per slice
   __shared__ __attribute__((aligned(16))) float xs[TM * kMRow];
   __shared__ __attribute__((aligned(16))) float ys[TN * kMRow];
-  const int64_t id = xcd_chunk(flat_block(), per);
+  // With a square causal matrix row tile m holds the column tiles that reach
+  // the diagonal, kQ (m + 1) of them (TI >= TJ) or m / kB + 1 (TI < TJ).
+  constexpr int kQ = TI >= TJ ? TI / TJ : 1, kB = TI >= TJ ? 1 : TJ / TI;
+  const int64_t pos = flat_block();
+  if (pos >= 8 * per) {
+    // causal == 1: workgroups past the tiles fill what lies to their right,
+    // kFillRows rows each.
+    const int nf = (p.Qb + kFillRows - 1) / kFillRows;
+    const int64_t f = pos - 8 * per, slab = f / nf;
+    if (slab * slab_tiles >= tiles) return;
+    float* o = p.scores + slab * p.Qb * p.Kb;
+    const bool wide = p.Kb % 4 == 0 && (uintptr_t)p.scores % 16 == 0;
+    for (int r = threadIdx.x >> 6; r < kFillRows; r += 4) {
+      const int i = (int)(f - slab * nf) * kFillRows + r, m = i / TI;
+      if (i >= p.Qb) return;
+      float* row = o + (int64_t)i * p.Kb;
+      int j = (TI >= TJ ? kQ * (m + 1) : m / kB + 1) * TJ;
+      if (wide) {
+        for (j += 4 * (threadIdx.x & 63); j < p.Kb; j += 256)
+          *reinterpret_cast<float4*>(row + j) = float4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      } else {
+        for (j += threadIdx.x & 63; j < p.Kb; j += 64) row[j] = -INFINITY;
+      }
+    }
+    return;
+  }
+  const int64_t id = xcd_chunk(pos, per);
   if (id >= tiles) return;
   const int64_t bg = id / slab_tiles;
   const int t = (int)(id - bg * slab_tiles);
   int ti, tj;
   const bool tri = slab_tiles != (int64_t)nti * ntj;
   if (tri) {
-    // Qb == Kb: row tile m holds the column tiles that reach the diagonal,
-    // kQ (m + 1) of them (TI >= TJ) or m / kB + 1 (TI < TJ), and the tiles
-    // before it are counted by `before`.
-    constexpr int kQ = TI >= TJ ? TI / TJ : 1, kB = TI >= TJ ? 1 : TJ / TI;
+    // `before` counts the tiles of the row tiles before m.
     auto before = [](int m) {
       const int64_t a = m / kB, r = m - a * kB;
       return kQ * (kB * (a * (a + 1) / 2) + r * (a + 1));
@@ -934,14 +967,8 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
       }
     return;
   }
-  if (tri && p.causal == 1 && j0 + TJ > i0 + TI - 1) {
-    // The row tile's last column tile also fills what lies to its right.
-    const int rows = p.Qb - i0 < TI ? p.Qb - i0 : TI;
-    for (int r = tid >> 6; r < rows; r += 4)
-      for (int j = j0 + TJ + lane; j < p.Kb; j += 64) out[(int64_t)(i0 + r) * p.Kb + j] = -INFINITY;
-  }
   // A wave whose outputs all lie above the diagonal or outside the matrix only stages.
-  const int iw = i0 + wr * 32 * RA / PQ, jw = j0 + wc * 64 / PK;
+  const int iw = i0 + wr * 32 * RA / PQ, jw = j0 + wc * 32 * RA / PK;
   const bool live = iw < p.Qb && jw < p.Kb && !(p.causal && jw > iw + 32 * RA / PQ - 1);
   const float* qsrc = p.qp + (bg * p.Qb + i0) * PQ * (int64_t)p.P;
   const float* ksrc = p.kp + (bg * p.Kb + j0) * PK * (int64_t)p.P;
@@ -975,28 +1002,28 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
 #pragma unroll
     for (int u = 0; u < YL; ++u) stage_even_odd(ys, (tid >> 3) + 32 * u, c4, yv[u]);
   };
-  f32x16_t acc[RA][2];
+  f32x16_t acc[RA][RA];
 #pragma unroll
   for (int a = 0; a < RA; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < RA; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
   const int xoff = (wr * 32 * RA + (lane & 31)) * kMRow + 4 * (lane >> 5);
-  const int yoff = (wc * 64 + (lane & 31)) * kMRow + 4 * (lane >> 5);
+  const int yoff = (wc * 32 * RA + (lane & 31)) * kMRow + 4 * (lane >> 5);
   // Pairs of e from e = 8 g of the slice (4 of them, or 2 in a tail).
   auto group = [&](int g, auto steps) {
-    f32x4_t x[RA], y[2];
+    f32x4_t x[RA], y[RA];
 #pragma unroll
     for (int a = 0; a < RA; ++a) x[a] = *reinterpret_cast<const f32x4_t*>(xs + xoff + 32 * a * kMRow + 8 * g);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) y[b] = *reinterpret_cast<const f32x4_t*>(ys + yoff + 32 * b * kMRow + 8 * g);
+    for (int b = 0; b < RA; ++b) y[b] = *reinterpret_cast<const f32x4_t*>(ys + yoff + 32 * b * kMRow + 8 * g);
 #pragma unroll
     for (int s = 0; s < decltype(steps)::value; ++s)
 #pragma unroll
       for (int a = 0; a < RA; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = mfma_f32(x[a][s], y[b][s], acc[a][b]);
+        for (int b = 0; b < RA; ++b) acc[a][b] = mfma_f32(x[a][s], y[b][s], acc[a][b]);
   };
   load_slice(0);
   int e0 = 0;
@@ -1022,8 +1049,8 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
   if (!live) {
     // Above the diagonal inside a computed tile (or outside the matrix).
     if (p.causal == 1)
-      for (int e = lane; e < (32 * RA / PQ) * (64 / PK); e += 64) {
-        const int i = iw + e / (64 / PK), j = jw + e % (64 / PK);
+      for (int e = lane; e < (32 * RA / PQ) * (32 * RA / PK); e += 64) {
+        const int i = iw + e / (32 * RA / PK), j = jw + e % (32 * RA / PK);
         if (i < p.Qb && j < p.Kb) out[(int64_t)i * p.Kb + j] = -INFINITY;
       }
     return;
@@ -1033,7 +1060,7 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
 #pragma unroll
   for (int a = 0; a < RA; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < RA; ++b)
 #pragma unroll
       for (int r0 = 0; r0 < 16; r0 += GS) {
         const float first = acc[a][b][r0];
@@ -1056,7 +1083,7 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
 #pragma unroll
     for (int a = 0; a < RA; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+      for (int b = 0; b < RA; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float x = acc[a][b][r];
@@ -1064,8 +1091,8 @@ __global__ __launch_bounds__(256, RA == 1 ? 4 : PQ * PK >= 16 ? 3 : 2) void gate
         }
     if (__ballot(negative) == 0) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // other lanes stored these scores above
-    for (int e = lane; e < (32 * RA / PQ) * (64 / PK); e += 64) {
-      const int i = iw + e / (64 / PK), j = jw + e % (64 / PK);
+    for (int e = lane; e < (32 * RA / PQ) * (32 * RA / PK); e += 64) {
+      const int i = iw + e / (32 * RA / PK), j = jw + e % (32 * RA / PK);
       if (i < p.Qb && j < p.Kb && (!p.causal || j <= i)) out[(int64_t)i * p.Kb + j] = score_in_order(p, bg, i, j);
     }
   }
@@ -2061,25 +2088,27 @@ extern "C" int spruce_gate_scores(const float* qp, const float* kp, int64_t BG, 
   if (!tri && causal == 2) p.causal = 1;
   auto pow2 = [](int64_t n) { return n == 1 || n == 2 || n == 4 || n == 8; };
   if (pow2(Pq) && pow2(Pk)) {
-    const int64_t ntj = (Kb * Pk + 127) / 128;
-    // Tiles of one slab at row tiles of TM prototype rows: with a square
-    // causal matrix only the tiles that reach the diagonal.
+    // Tiles of one slab, of TM x TM prototype rows: with a square causal matrix
+    // only those that reach the diagonal.
     auto slab = [&](int64_t TM) {
-      const int64_t nti = (Qb * Pq + TM - 1) / TM, TI = TM / Pq, TJ = 128 / Pk;
+      const int64_t nti = (Qb * Pq + TM - 1) / TM, ntj = (Kb * Pk + TM - 1) / TM, TI = TM / Pq, TJ = TM / Pk;
       if (!causal || Qb != Kb) return nti * ntj;
       const int64_t q = TI >= TJ ? TI / TJ : 1, b = TI >= TJ ? 1 : TJ / TI, a = nti / b, r = nti - a * b;
       return q * (b * (a * (a + 1) / 2) + r * (a + 1));
     };
-    SPRUCE_REQUIRE((Qb * Pq + 63) / 64 * ntj < ((int64_t)1 << 31), "score matrix too large");
+    SPRUCE_REQUIRE((Qb * Pq + 127) / 128 * ((Kb * Pk + 127) / 128) < ((int64_t)1 << 31), "score matrix too large");
     // 128-row tiles once they give every CU two workgroups; smaller grids take 64-row tiles.
     const bool big = BG * slab(128) >= 512;
-    const int64_t nti = (Qb * Pq + (big ? 127 : 63)) / (big ? 128 : 64);
-    const int64_t per_slab = slab(big ? 128 : 64), tiles = BG * per_slab;
+    const int64_t TM = big ? 128 : 64;
+    const int64_t nti = (Qb * Pq + TM - 1) / TM, ntj = (Kb * Pk + TM - 1) / TM;
+    const int64_t per_slab = slab(TM), tiles = BG * per_slab;
     int64_t per = (tiles + 7) / 8;
     if (8 * per > kGridX) per = (per + kGridX / 8 - 1) / (kGridX / 8) * (kGridX / 8);  // whole rows of the grid
     SPRUCE_REQUIRE(8 * per < ((int64_t)1 << 31), "score matrix too large");
+    const int64_t fill = p.causal == 1 && per_slab != nti * ntj ? BG * ((Qb + kFillRows - 1) / kFillRows) : 0;
+    SPRUCE_REQUIRE(8 * per + fill < ((int64_t)1 << 31), "score matrix too large");
     auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, flat_grid(8 * per), dim3(256), 0, (hipStream_t)stream, p, (int)nti, (int)ntj, per_slab,
+      hipLaunchKernelGGL(kernel, flat_grid(8 * per + fill), dim3(256), 0, (hipStream_t)stream, p, (int)nti, (int)ntj, per_slab,
                          tiles, per);
     };
     auto pick = [&](auto pq, auto pk) {

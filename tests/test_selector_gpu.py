@@ -455,6 +455,21 @@ def test_matrix_scores_keep_the_sign_of_zero(Pq, Pk):
     assert negative > 100
 
 
+@pytest.mark.parametrize("Pq,Pk", [(1, 1), (1, 2), (2, 4), (8, 1), (1, 8), (8, 8)])
+def test_causal_scores_fill_what_no_tile_covers(Pq, Pk):
+    # Square causal matrices of several tiles: the columns right of a row's
+    # tiles are filled 16 rows a workgroup, 16 bytes at a time where rows are
+    # aligned; memory that held NaN before.
+    gen = torch.Generator().manual_seed(Pq * 10 + Pk)
+    for S, n in ((3, 65), (2, 130), (1, 203), (2, 260), (70, 64)):
+        qp = torch.randn(S, n, Pq, 4, generator=gen)
+        kp = torch.randn(S, n, Pk, 4, generator=gen)
+        torch.full((S, n, n), float("nan"), device=DEV)   # freed: the output takes its place
+        print(f"causal fill {Pq} x {Pk} S={S} n={n}", flush=True)
+        got = _np(gate_scores(qp.to(DEV), kp.to(DEV), causal=True))
+        np.testing.assert_array_equal(got, osel.scores(qp.numpy(), kp.numpy(), causal=True))
+
+
 @pytest.mark.parametrize("Pq,Pk,P", [(8, 8, 4), (1, 3, 216)])
 def test_scores_past_two_to_the_32_threads(Pq, Pk, P):
     # Grids of more than 2^32 threads: the matrix cores (a workgroup per 16 x
