@@ -590,10 +590,10 @@ __device__ __forceinline__ f32x4_t widen4(const ProjRowsSeg<TIn>&, V w) {
   }
 }
 
-// Projections as one matrix product: a workgroup of 2 x 2 waves covers
-// 64 RA x 128 outputs, each wave 32 RA x 64, in slices of 32 d (the next
-// slice's loads are in flight during the current one's products).  blockIdx.z is the layer: `rows` rows of x, its own [D, P]
-// weights.
+// Projections as one matrix product: a workgroup of 4 / WC x WC waves covers
+// 32 RA (4 / WC) x 64 WC outputs, each wave 32 RA x 64, in slices of 32 d (the
+// next slice's loads are in flight during the current one's products).
+// blockIdx.z is the layer: `rows` rows of x, its own [D, P] weights.
 // IL: rows are (node, prototype) pairs with ilk prototypes per node, and out
 // is [nodes, P/4, ilk, 4] (each node's prototypes interleaved by 4-column
 // group) instead of [N, P].  The operands then change sides (A = columns of
@@ -612,16 +612,17 @@ __device__ __forceinline__ f32x4_t widen4(const ProjRowsSeg<TIn>&, V w) {
 // P = 64: 64 rows 5.7 and 6.6, 8192 rows 6.6 and 7.3, 16383 rows (256 tiles)
 // 7.0 and 6.8.
 constexpr int kMfmaProjectRows = 8192, kMfmaProjectTiles = 256, kMfmaPairRows = 16384;
-template <int RA, typename Rows, bool IL>
+template <int RA, int WC, typename Rows, bool IL>
 __global__ __launch_bounds__(256, RA == 2 ? 3 : 4) void project_mfma_kernel(const Rows src, const float* __restrict__ w,
                                                                             int64_t rows, int D, int P,
                                                                             float* __restrict__ out, int ilk) {
-  constexpr int R = IL ? 128 : 64 * RA, C = IL ? 64 * RA : 128;  // rows of x, columns of w per workgroup
+  constexpr int TA = 32 * RA * (4 / WC), TB = 64 * WC;     // sides A and B of a workgroup's tile
+  constexpr int R = IL ? TB : TA, C = IL ? TA : TB;        // rows of x, columns of w per workgroup
   constexpr int XL = R * kMS / 4 / 256, WL = C * kMS / 4 / 256;  // groups of 4 d per thread per slice
   __shared__ __attribute__((aligned(16))) float xs[R * kMRow];
   __shared__ __attribute__((aligned(16))) float ws[C * kMRow];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wr = __builtin_amdgcn_readfirstlane(tid >> 7), wc = __builtin_amdgcn_readfirstlane((tid >> 6) & 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave / WC, wc = wave % WC;
   const int64_t n0 = (int64_t)blockIdx.x * R, base = (int64_t)blockIdx.z * rows;
   const int j0 = blockIdx.y * C;
   const int c4 = tid & 7;
@@ -740,8 +741,19 @@ int launch_project_mfma(const Rows& src, const float* w, int64_t L, int64_t rows
                        ilk);
     return check_launch("project_mfma_kernel");
   };
-  if (il) return big >= 512 ? go(project_mfma_kernel<2, Rows, true>, 128, 128) : go(project_mfma_kernel<1, Rows, true>, 128, 64);
-  return big >= 512 ? go(project_mfma_kernel<2, Rows, false>, 128, 128) : go(project_mfma_kernel<1, Rows, false>, 64, 128);
+  // An odd number of 64-column pieces leaves half of a 128-column tile empty:
+  // 64-column tiles there, once 64 x 128 ones (il: 128 x 128) would be more than
+  // one a CU.  D = 128, bf16, P = 64: 16,800 rows 15.9 -> 11.3 us (4064 rows 10.8
+  // and 11.5), 122,880 rows 48.7 -> 30.0, interleaved 46.5 -> 28.4; P = 192: 88.7
+  // -> 72.2 and 83.1 -> 68.9.
+  const bool odd = (P + 63) / 64 % 2 != 0;
+  const bool narrow = odd && L * ((rows + 63) / 64) * ((P + 127) / 128) > 256;
+  if (il)
+    return big >= 512 && !odd ? go(project_mfma_kernel<2, 2, Rows, true>, 128, 128)
+                                 : go(project_mfma_kernel<1, 2, Rows, true>, 128, 64);
+  if (narrow) return go(project_mfma_kernel<1, 1, Rows, false>, 128, 64);
+  return big >= 512 ? go(project_mfma_kernel<2, 2, Rows, false>, 128, 128)
+                    : go(project_mfma_kernel<1, 2, Rows, false>, 64, 128);
 }
 
 // MaxSim scores over a tile of 16 query blocks x 64 key blocks: lane = key

@@ -487,7 +487,8 @@ def test_scores_past_two_to_the_32_threads(Pq, Pk, P):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("L,S,nodes,Pk,D,P", [
-    (1, 1, [1], 1, 4, 4), (3, 2, [37, 19, 1], 8, 36, 64), (2, 1, [70], 4, 128, 132), (2, 3, [1500, 750, 5], 8, 32, 260)])
+    (1, 1, [1], 1, 4, 4), (3, 2, [37, 19, 1], 8, 36, 64), (2, 1, [70], 4, 128, 132), (2, 3, [1500, 750, 5], 8, 32, 260),
+    (1, 1, [2048], 8, 36, 64), (1, 1, [2049], 8, 36, 64), (1, 2, [4099], 8, 32, 192), (3, 1, [700], 8, 32, 20)])
 def test_projection_of_layers_equals_each_layer(dtype, L, S, nodes, Pk, D, P):
     # One launch over layers and levels (both tile heights, row and column
     # remainders, tails of the 32-wide slices, both output layouts) against
