@@ -1006,7 +1006,13 @@ extern "C" int spruce_tree_traverse(const float* qp, const float* kp, int64_t S,
     hipLaunchKernelGGL(kernel, grid, dim3(64), lds, (hipStream_t)stream, p);
   };
   // Matrix-core scoring, with the key group stride fixed where it is known:
-  // as many key prototypes as query prototypes interleaved, or rows.
+  // as many key prototypes as query prototypes interleaved, or rows.  Of the
+  // rows layout every lane reads a line of its own, which in large grids the
+  // caches bound: up to 1280 rows there (five waves a CU), VALU chains past
+  // that.  4 slabs, beam 16, 8 x 8 prototypes of 128 dims, matrix cores and
+  // VALU: 64 leaves 21 and 43 us, 300 105 and 116, 340 138 and 126, 1000 548
+  // and 407, 2048 1326 and 938 (4 x 4: 51 and 54, 68 and 64, 272 and 229, 656
+  // and 558).
   auto mfma = [&](auto pq, auto dim) {
     constexpr int Q = decltype(pq)::value, D = decltype(dim)::value;
     if (il && Pk == Q)
@@ -1017,10 +1023,11 @@ extern "C" int spruce_tree_traverse(const float* qp, const float* kp, int64_t S,
       go(tree_traverse_kernel<Q, D, 0>);
   };
   using std::integral_constant;
-  if (Pq == 8 && pd == 128) mfma(integral_constant<int, 8>{}, integral_constant<int, 128>{});
-  else if (Pq == 8 && pd == 64) mfma(integral_constant<int, 8>{}, integral_constant<int, 64>{});
-  else if (Pq == 4 && pd == 128) mfma(integral_constant<int, 4>{}, integral_constant<int, 128>{});
-  else if (Pq == 4 && pd == 64) mfma(integral_constant<int, 4>{}, integral_constant<int, 64>{});
+  const bool cores = il || S * qb <= 1280;
+  if (cores && Pq == 8 && pd == 128) mfma(integral_constant<int, 8>{}, integral_constant<int, 128>{});
+  else if (cores && Pq == 8 && pd == 64) mfma(integral_constant<int, 8>{}, integral_constant<int, 64>{});
+  else if (cores && Pq == 4 && pd == 128) mfma(integral_constant<int, 4>{}, integral_constant<int, 128>{});
+  else if (cores && Pq == 4 && pd == 64) mfma(integral_constant<int, 4>{}, integral_constant<int, 64>{});
   else if (Pq == 8) go(tree_traverse_kernel<8>);
   else if (Pq == 4) go(tree_traverse_kernel<4>);
   else if (Pq == 2) go(tree_traverse_kernel<2>);
