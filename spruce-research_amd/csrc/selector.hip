@@ -900,9 +900,9 @@ __device__ __forceinline__ float dpp_max(float x) {
 // score (every pair a dependent chain whose operands come through the cache)
 // -> 0.319 ms.  One query and two key prototypes, 4 slabs of 1024 blocks:
 // 31.9 (VALU, 2 x 4 x 2 outputs a thread) -> 23.8 us with 64 x 128 tiles in
-// small grids; launch to launch in a captured graph 21.5 -> 18.9 us with the
-// 64 x 64 ones, of which a wave's outputs and code are half, most of a short
-// kernel (one prototype of 32 dims, 4 slabs of 64 blocks: 5.1 -> 3.9 us).
+// small grids, -> 21.5 us with the 64 x 64 ones, of which a wave's outputs and
+// code are half, most of a short kernel (one prototype of 32 dims, 4 slabs of
+// 64 blocks, launch to launch in a captured graph: 5.1 -> 3.9 us).
 //
 // causal == 1 with Qb == Kb: what lies right of a row's tiles is filled by
 // workgroups of its own past the tiles, 16 rows each (filled by the row's last
