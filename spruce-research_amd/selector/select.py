@@ -146,9 +146,8 @@ def project_levels(levels, W, interleaved=False):
     the tree traversal reads fastest."""
     if not levels:
         raise ValueError("levels must not be empty")
-    for t in levels:
-        if t.dim() != 4:
-            raise ValueError("levels must be [S, n, P, D] with one S, P, D and dtype")
+    if any(t.dim() != 4 for t in levels):
+        raise ValueError("levels must be [S, n, P, D] with one S, P, D and dtype")
     if W.dim() != 2 or W.shape[0] != levels[0].shape[-1]:
         raise ValueError(f"shape mismatch: levels [..., {levels[0].shape[-1]}] @ W {tuple(W.shape)}")
     return project_layers([t.unsqueeze(0) for t in levels], W.unsqueeze(0), interleaved=interleaved)[0]
@@ -161,12 +160,13 @@ def project_layers(levels, W, interleaved=False):
     values of L ``project_levels`` calls."""
     if not levels:
         raise ValueError("levels must not be empty")
+    L, S, _, P, D = levels[0].shape if levels[0].dim() == 5 else (None,) * 5
+    dtype = levels[0].dtype
     for t in levels:
         _cuda(t, "levels")
-        if t.dim() != 5 or t.shape[:2] != levels[0].shape[:2] or t.shape[3:] != levels[0].shape[3:] or \
-                t.dtype != levels[0].dtype:
+        n = t.shape   # compared one by one: a slice of a shape costs as much as all of this
+        if len(n) != 5 or n[0] != L or n[1] != S or n[3] != P or n[4] != D or t.dtype != dtype:
             raise ValueError("levels must be [L, S, n, P, D] with one L, S, P, D and dtype")
-    L, S, _, P, D = levels[0].shape
     if W.dim() != 3 or W.shape[:2] != (L, D):
         raise ValueError(f"shape mismatch: levels [..., {D}] of {L} layers @ W {tuple(W.shape)}")
     W = W.to(device=levels[0].device, dtype=torch.float32).contiguous()
